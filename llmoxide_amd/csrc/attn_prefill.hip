@@ -12,9 +12,9 @@
 //                 S^T accumulators (no shuffle: computing the transpose makes
 //                 each lane own one query column, so softmax is mostly in-lane)
 //
-// Three kernels share these tiles.  attn_prefill_kernel: workgroup = 4 waves x
-// 32 query rows, of one query head or of 2-4 heads that share a kv head
-// (head_dim >= 256), two workgroups per CU below head_dim 256.  The ping-pong
+// Three kernels here share these tiles (head_dim 64 and 128; 256 and 512 are
+// attn_prefill_wide.hip's).  attn_prefill_kernel: workgroup = 4 waves x 32
+// query rows of one query head, two workgroups per CU.  The ping-pong
 // kernel (head_dim 128, long batches): 8 waves x 32 rows, one workgroup per
 // CU, the two waves of each SIMD kept half a tile apart so one's MFMAs run
 // beside the other's softmax.  The key-halves kernel (short batches): 64
@@ -29,84 +29,19 @@
 #include <cstdlib>
 #include <cstring>
 
-#include "common.hpp"
-
-
+#include "attn_prefill.hpp"
 
 namespace lmx {
 
-struct PrefillArgs {
-    const void* q;
-    const f16* k;
-    const f16* v;
-    const f16* k_cur;
-    const f16* v_cur;
-    float* out;
-    const float* gate;  // NULL, or the output gate: out *= sigmoid(gate[row * gate_stride + d])
-    int q_stride, gate_stride;
-    int H, Hkv, G, kv_dim;
-    int base_pos, window, n_tokens, bidi;
-    int n_qtiles;
-    int gp;  // attn_prefill_kernel: query heads per workgroup (1, 2 or 4, dividing G)
-    uint32_t w_magic;  // p % window == ring_slot(p, window, w_magic, w_shift)
-    int w_shift;
-    float c;  // scale * log2(e)
-    // Key-range split (attn_prefill_kernel only): n_split > 1 writes each
-    // split's unnormalized o and its (m, l) to part_o / part_ml for
-    // prefill_merge_kernel.
-    int n_split;
-    float* part_o;   // [n_split][t][H][hd]
-    float* part_ml;  // [n_split][t][H][2]
-};
-
 constexpr int kPfBM = 128;  // query rows per workgroup
 constexpr int kPfCus = 256;  // compute units of the target (MI355X)
-// Keys per LDS tile: 64, or 32 at head_dim >= 256 (the register prefetch of
-// the next tile and the o accumulators share one register file).
-template <int HD>
-constexpr int pf_bn() { return HD >= 256 ? 32 : 64; }
-// Wave pairs at head_dim 512: a wave cannot hold a 32-row block's Q and its
-// 32 x 512 fp32 output in registers, so two waves share each block, one per
-// half of the head's dims.  Each holds its half of Q and of the output (the
-// register budget of head_dim 256), forms the partial S over its 256 dims,
-// and the two partials are summed through LDS; both waves then hold the
-// same scores (a + b = b + a in IEEE arithmetic), run the same softmax, and
-// accumulate P V for their own half.  The MFMA work is that of one pass.
-template <int HD>
-constexpr bool pf_pair() { return HD >= 512; }
-constexpr float kRescaleSlack = 8.f;  // log2 units a running max may lag by
-
-// attn.wgsl:52-66
-__device__ __forceinline__ int vis_lo(int pos, int w) { return (w && pos + 1 > w) ? pos + 1 - w : 0; }
-__device__ __forceinline__ int vis_hi(int pos, int w, int bidi, int end) {
-    if (!bidi) return pos;
-    return w ? min(end, pos + w - 1) : end;
-}
-
 // S^T - mb = K Q^T - mb for KB 32-key blocks of a K tile in LDS (rows of
 // KPAD halfs), Q^T in registers as the B operand.  The K operand reads run
 // QK_DEPTH ahead of the MFMAs (the compiler's own schedule kept one or two
 // in flight, so every MFMA waited out most of an LDS round trip); the
-// (k-step, block) order alternates the KB accumulator chains.  Depth 4 at
-// head_dim <= 128 (6 spills in the 128-row kernel), QK_DEPTH_HD256 at 256,
-// where one wave per SIMD has the registers (measured: depth 4 +2-3% at
-// S = 8192, +7% on Gemma hd 256 global 4k; depth 6 a further +2-3% there),
-// and 2 at head_dim 512, whose Q alone takes 128 registers.
-#ifndef LMX_QK_DEPTH_HD256
-#define LMX_QK_DEPTH_HD256 8
-#endif
-template <int HD>
-constexpr int qk_depth() { return HD >= 512 ? 2 : (HD >= 256 ? LMX_QK_DEPTH_HD256 : 4); }
-// The wave pairs of head_dim 512 hold twice the K/V prefetch of head_dim 256
-// in registers: shallower operand rings keep them out of scratch.
-#ifndef LMX_PAIR_QK_DEPTH
-#define LMX_PAIR_QK_DEPTH 2
-#endif
-#ifndef LMX_PAIR_PV_DEPTH
-#define LMX_PAIR_PV_DEPTH 1
-#endif
-constexpr int kPairQkDepth = LMX_PAIR_QK_DEPTH;
-constexpr int kPairPvDepth = LMX_PAIR_PV_DEPTH;
+// (k-step, block) order alternates the KB accumulator chains.  Depth 4: 6
+// spills in the 128-row kernel (+2-3% at S = 8192 when measured).
+constexpr int kQkDepth = 4;
 //
 // EXACT: Q holds the caller's f16 values and the scores are scaled by
 // c = scale * log2(e) in fp32 after the MFMAs (one FMA per score).  Else c
@@ -125,16 +60,15 @@ constexpr int kPairPvDepth = LMX_PAIR_PV_DEPTH;
 // one rounding of q moves scores by ~1e-2 in log2 units).  The row scaling
 // keeps hi and the residuals of all but tiny elements in f16's normal range,
 // where they keep their full 11 bits.  ql(ks) returns the residual's fragment
-// of k-step ks (from LDS, or recomputed from the fp32 query in memory where
-// no LDS is left).
+// of k-step ks (from LDS).
 struct NoQlo {
     __device__ f16x8 operator()(int) const { return f16x8{}; }
 };
-template <int HD, int KB, int KPAD, bool EXACT, bool QLO = false, typename QL = NoQlo, int DEP = qk_depth<HD>()>
+template <int HD, int KB, int KPAD, bool EXACT, bool QLO = false, typename QL = NoQlo>
 __device__ __forceinline__ void qk_tile(const f16* Ks, const f16x8 (&qf)[HD / 16], f32x16 (&s)[KB], float mb,
                                         float c, int l32, int hh, const QL& ql = QL{}) {
     constexpr int KSTEPS = HD / 16, NQ = KSTEPS * KB;
-    constexpr int D = DEP < NQ ? DEP : NQ;
+    constexpr int D = kQkDepth < NQ ? kQkDepth : NQ;
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
@@ -167,20 +101,6 @@ __device__ __forceinline__ void qk_tile(const f16* Ks, const f16x8 (&qf)[HD / 16
     }
 }
 
-// Q fragments as values defined here, not the registers of their loads (an
-// f16 query's conversions fold away): otherwise the waitcnt pass counts Q's
-// loads as possibly pending inside the key loop and puts vmcnt(n) waits
-// between the score MFMAs, which drain the K/V prefetch of later tiles.
-template <int N>
-__device__ __forceinline__ void settle_q(f16x8 (&qf)[N]) {
-#pragma unroll
-    for (int i = 0; i < N; ++i) asm volatile("" : "+v"(qf[i]));
-}
-
-// s_waitcnt vmcnt(0) as an instruction the compiler's waitcnt pass sees
-// (inline assembly it does not): every load issued before it is complete.
-__device__ __forceinline__ void drain_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }
-
 // A raw buffer resource over p (dword 3 = 0x00020000: 32-bit data format, the
 // form raw buffer loads take on gfx9 parts) with 2^31 - 1 bytes of range,
 // which the rows of one K/V tile never leave.  p must be wave-uniform: it is
@@ -198,30 +118,23 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* p) {
 // the common causal case; its addressing is compiled without the general
 // path's branches (which cost the main loop 3-8% in registers and schedule).
 template <typename QT, int HD, bool LIN>
-__global__ __launch_bounds__(256, HD > 128 ? 1 : 2) void attn_prefill_kernel(PrefillArgs a) {
+__global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PrefillArgs a) {
     constexpr bool kExact = sizeof(QT) == 2;  // f16 queries: scale applied in fp32 (qk_tile)
-    constexpr int BN = pf_bn<HD>();
-    constexpr bool kPair = pf_pair<HD>();
-    constexpr int QD = kPair ? HD / 2 : HD;  // Q dims a wave holds (its half, kPair)
-    constexpr int HDV = QD;          // output dims a wave accumulates
+    static_assert(HD <= 128, "larger heads: attn_prefill_wide_kernel");
+    constexpr int BN = 64;
     constexpr int KB = BN / 32;      // 32-key MFMA blocks per tile
-    constexpr int PST = BN / 16;     // 16-key P.V k-steps per tile
-    constexpr int KSTEPS = QD / 16;  // MFMA k-steps over the wave's dims
-    constexpr int NB = HDV / 32;     // 32-dim output blocks
+    constexpr int KSTEPS = HD / 16;  // MFMA k-steps over head_dim
+    constexpr int NB = HD / 32;      // 32-dim output blocks
     constexpr int KPAD = HD + 8;     // K_s row stride (halfs)
     constexpr int VPAD = BN + 4;     // Vt_s row stride (halfs), 8-byte aligned rows
     __shared__ __attribute__((aligned(16))) f16 K_s[2 * BN * KPAD];   // two stages
     __shared__ __attribute__((aligned(16))) f16 Vt_s[2 * HD * VPAD];
-    // kPair: each wave's partial scores, 16 floats a lane as four f32x4
-    // planes of 64 lanes (conflict-free 16-byte accesses)
-    __shared__ __attribute__((aligned(16))) float X_s[kPair ? 4 * 16 * 64 : 4];
     // fp32 queries: the residual of q*c after its f16 rounding, one padded row
     // per query (the stride spreads a read's 32 rows over the banks as K_s's
-    // does); at head_dim 512 the LDS is full and it is recomputed instead.
+    // does).
     constexpr bool kQlo = !kExact;
-    constexpr bool kQloLds = kQlo && HD <= 256;
     constexpr int QLPAD = HD + 8;
-    __shared__ __attribute__((aligned(16))) f16 QL_s[kQloLds ? 4 * 32 * QLPAD : 8];
+    __shared__ __attribute__((aligned(16))) f16 QL_s[kQlo ? 4 * 32 * QLPAD : 8];
 
     // ---- which (heads, query tile, key split) this workgroup owns.  The gp
     // query heads of a workgroup share kv head kvh; each takes 4 / gp waves,
@@ -241,7 +154,7 @@ __global__ __launch_bounds__(256, HD > 128 ? 1 : 2) void attn_prefill_kernel(Pre
     // tile with a light one instead of two of nearly the same weight.
     const int pos = rem / (hgroups * n_split);
     const int half = (a.n_qtiles + 1) / 2;
-    const bool fold = HD <= 128 && nblk <= 2 * kPfCus;
+    const bool fold = nblk <= 2 * kPfCus;
     const int qt = (fold && pos >= half) ? pos - half : a.n_qtiles - 1 - pos;
     const int rem2 = rem % (hgroups * n_split);
     const int sp = rem2 % n_split;
@@ -252,17 +165,13 @@ __global__ __launch_bounds__(256, HD > 128 ? 1 : 2) void attn_prefill_kernel(Pre
     // buffer loads)
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, hh = lane >> 5;
-    // kPair: waves w and w ^ 2 share a 32-row block, dims [dh * QD, + QD)
-    // each; otherwise every wave has its own block of all the dims.
-    const int dh = kPair ? wave >> 1 : 0;
-    const int wr = kPair ? wave & 1 : wave;  // the wave's row block
-    const int wph = (kPair ? 2 : 4) / gp;    // row blocks per query head
+    const int wph = 4 / gp;                  // row blocks per query head
     const int bm = 32 * wph;                 // query rows per head
-    const int h = kvh * a.G + (rem2 / n_split) * gp + wr / wph;  // this wave's head
+    const int h = kvh * a.G + (rem2 / n_split) * gp + wave / wph;  // this wave's head
     const int t = a.n_tokens, base = a.base_pos, w = a.window;
     const int end = base + t - 1;
     const int q0 = qt * bm;
-    const int qw0 = q0 + (wr % wph) * 32;
+    const int qw0 = q0 + (wave % wph) * 32;
 
     // ---- this lane's query (column l32 of the wave's S^T tiles)
     const int qrow = qw0 + l32;
@@ -276,9 +185,9 @@ __global__ __launch_bounds__(256, HD > 128 ? 1 : 2) void attn_prefill_kernel(Pre
     // residual is the second operand (kQlo); an f16 query is used as given and
     // qk_tile scales its scores.
     f16x8 qf[KSTEPS];
-    const size_t qoff = ((size_t)(qvalid ? qrow : 0) * a.H + h) * a.q_stride + dh * QD + 8 * hh;
+    const size_t qoff = ((size_t)(qvalid ? qrow : 0) * a.H + h) * a.q_stride + 8 * hh;
     const float* qrow32 = reinterpret_cast<const float*>(a.q) + qoff;
-    f16* ql_row = &QL_s[kQloLds ? (wave * 32 + l32) * QLPAD + 8 * hh : 0];
+    f16* ql_row = &QL_s[kQlo ? (wave * 32 + l32) * QLPAD + 8 * hh : 0];
     // fp32 queries: c 2^S folded into Q (the row's largest |x c 2^S| in
     // [2^14, 2^15); 2^S = 1 for an all-zero or non-finite row), and the
     // scores scaled back by c_sc = 2^-S; f16 queries: Q as given, c_sc = c.
@@ -333,7 +242,7 @@ __global__ __launch_bounds__(256, HD > 128 ? 1 : 2) void attn_prefill_kernel(Pre
                     qf[ks][j] = (f16)y[j];
                 }
                 asm volatile("" : "+v"(qf[ks]));
-                if constexpr (kQloLds) {
+                {
                     f16x8 lo;
 #pragma unroll
                     for (int j = 0; j < 8; ++j) lo[j] = (f16)(y[j] - (float)qf[ks][j]);
@@ -346,18 +255,8 @@ __global__ __launch_bounds__(256, HD > 128 ? 1 : 2) void attn_prefill_kernel(Pre
     // The residual's fragment of k-step ks (read after the first barrier of
     // the key loop, which orders the stores above before it).
     auto ql = [&](int ks) -> f16x8 {
-        if constexpr (kQloLds) {
+        if constexpr (kQlo) {
             return *reinterpret_cast<const f16x8*>(ql_row + ks * 16);
-        } else if constexpr (kQlo) {
-            const f32x4 x0 = *reinterpret_cast<const f32x4*>(qrow32 + ks * 16);
-            const f32x4 x1 = *reinterpret_cast<const f32x4*>(qrow32 + ks * 16 + 4);
-            f16x8 lo;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                lo[j] = (f16)(x0[j] * qc - (float)qf[ks][j]);
-                lo[4 + j] = (f16)(x1[j] * qc - (float)qf[ks][4 + j]);
-            }
-            return lo;
         } else {
             return f16x8{};
         }
@@ -391,9 +290,8 @@ __global__ __launch_bounds__(256, HD > 128 ? 1 : 2) void attn_prefill_kernel(Pre
     // banks once.  Consecutive dims would put lanes 8 rows apart, on two
     // banks (the row stride is 16 banks mod 32).
     constexpr int KCH = HD / 8;                   // 16-byte chunks per key row
-    constexpr int KCHV = HD / 8;                  // 16-byte chunks of a V row
     constexpr int KPT = BN * KCH / 256;           // K chunks per thread
-    constexpr int VPT = (KCHV * (BN / 4) + 255) / 256;  // V 4-key groups per thread
+    constexpr int VPT = (KCH * (BN / 4) + 255) / 256;  // V 4-key groups per thread
     static_assert(BN * KCH % 256 == 0, "K tile split");
     f16x8 rk[KPT];
     f16x8 rv[VPT][4];
@@ -450,7 +348,7 @@ __global__ __launch_bounds__(256, HD > 128 ? 1 : 2) void attn_prefill_kernel(Pre
                     f16x8, __builtin_amdgcn_raw_buffer_load_b128(rk_src, k_voff, i * (256 / KCH) * kvb, 0));
 #pragma unroll
             for (int i = 0; i < VPT; ++i) {
-                if (tid + 256 * i < KCHV * (BN / 4))
+                if (tid + 256 * i < KCH * (BN / 4))
 #pragma unroll
                     for (int u = 0; u < 4; ++u)
                         rv[i][u] = __builtin_bit_cast(
@@ -469,7 +367,7 @@ __global__ __launch_bounds__(256, HD > 128 ? 1 : 2) void attn_prefill_kernel(Pre
         for (int i = 0; i < VPT; ++i) {
             const int pr = tid + 256 * i;
             const int kg = pr % (BN / 4), dc = pr / (BN / 4);
-            if (pr < KCHV * (BN / 4))
+            if (pr < KCH * (BN / 4))
 #pragma unroll
                 for (int u = 0; u < 4; ++u)
                     rv[i][u] = *reinterpret_cast<const f16x8*>(vb + (size_t)(4 * kg + u) * a.kv_dim + dc * 8);
@@ -499,7 +397,7 @@ __global__ __launch_bounds__(256, HD > 128 ? 1 : 2) void attn_prefill_kernel(Pre
             for (int u = 0; u < 4; ++u) {
                 const int p = kt + 4 * kg + u;
                 f16x8 val = {};
-                if (pr < KCHV * (BN / 4) && p >= wg_lo && p <= wg_hi)
+                if (pr < KCH * (BN / 4) && p >= wg_lo && p <= wg_hi)
                     val = *reinterpret_cast<const f16x8*>(row_src(a.v, a.v_cur, p) + kvh * HD + dc * 8);
                 rv[i][u] = val;
             }
@@ -517,7 +415,7 @@ __global__ __launch_bounds__(256, HD > 128 ? 1 : 2) void attn_prefill_kernel(Pre
 #pragma unroll
         for (int i = 0; i < VPT; ++i) {
             const int pr = tid + 256 * i;
-            if (pr >= KCHV * (BN / 4)) continue;
+            if (pr >= KCH * (BN / 4)) continue;
             const int kg = pr % (BN / 4), dc = pr / (BN / 4);
 #pragma unroll
             for (int j = 0; j < 8; ++j)
@@ -540,41 +438,17 @@ __global__ __launch_bounds__(256, HD > 128 ? 1 : 2) void attn_prefill_kernel(Pre
         stash(stage);
         __syncthreads();
         if (kt + BN <= kt_stop) fetch(kt + BN);
-        // wave-uniform, and the same for both waves of a kPair block
-        const bool live = wave_live && kt <= wv_hi && kt + BN - 1 >= wv_lo;
-        if (!kPair && !live) continue;
+        if (!wave_live || kt > wv_hi || kt + BN - 1 < wv_lo) continue;  // wave-uniform
         const bool need_mask = !(kt >= wv_lo_max && kt + BN - 1 <= wv_hi_min);
         const f16* Ks = K_s + stage * (BN * KPAD);
-        const f16* Vts = Vt_s + stage * (HD * VPAD) + dh * HDV * VPAD;
+        const f16* Vts = Vt_s + stage * (HD * VPAD);
 
         // ---- S^T - m = K Q^T - m, two 32-key blocks.  The accumulators start
         //      at -mb (mb = the running max once one is set), so the scores
-        //      come out already shifted for exp2.  kPair: each wave's partial
-        //      over its dims, scaled (c_sc), goes through X_s; every wave
-        //      meets the barrier, live or not; the sum is then shifted by mb.
+        //      come out already shifted for exp2.
         float mb = m_run > -1e29f ? m_run : 0.f;
         f32x16 s[KB];
-        if constexpr (kPair) {
-            static_assert(KB == 1, "one 32-key block per tile in the pair exchange");
-            if (live) {
-                qk_tile<QD, KB, KPAD, true, kQlo, decltype(ql), kPairQkDepth>(Ks + dh * QD, qf, s, 0.f, c_sc, l32,
-                                                                              hh, ql);
-#pragma unroll
-                for (int g = 0; g < 4; ++g)
-                    *reinterpret_cast<f32x4*>(&X_s[((wave * 4 + g) * 64 + lane) * 4]) =
-                        f32x4{s[0][4 * g], s[0][4 * g + 1], s[0][4 * g + 2], s[0][4 * g + 3]};
-            }
-            __syncthreads();
-            if (!live) continue;
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const f32x4 o4 = *reinterpret_cast<const f32x4*>(&X_s[(((wave ^ 2) * 4 + g) * 64 + lane) * 4]);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) s[0][4 * g + j] = (s[0][4 * g + j] + o4[j]) - mb;
-            }
-        } else {
-            qk_tile<HD, KB, KPAD, true, kQlo>(Ks, qf, s, mb, c_sc, l32, hh, ql);
-        }
+        qk_tile<HD, KB, KPAD, true, kQlo>(Ks, qf, s, mb, c_sc, l32, hh, ql);
 
         // ---- mask, online softmax.  s[kb][i] is key
         //      kt + 32*kb + 8*(i/4) + 4*hh + i%4 for query qrow, minus mb.
@@ -663,10 +537,7 @@ __global__ __launch_bounds__(256, HD > 128 ? 1 : 2) void attn_prefill_kernel(Pre
                     va[st] = f16x8{v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
                 }
             };
-            // Operands PVD blocks ahead: 2 at head_dim >= 256, where one wave
-            // per SIMD waits out each LDS round trip (+1.2% on Gemma's 4k
-            // prefill; 3 measured the same), 1 below.
-            constexpr int PVD = kPair ? kPairPvDepth : (HD >= 256 ? 2 : 1);
+            constexpr int PVD = 1;  // operands one block ahead
             static_assert(PVD < NB, "operand ring");
             f16x8 va[PVD + 1][2];
 #pragma unroll
@@ -691,8 +562,8 @@ __global__ __launch_bounds__(256, HD > 128 ? 1 : 2) void attn_prefill_kernel(Pre
         // the split's partial: o as accumulated, and (m, l); an empty split
         // leaves m = -1e30, l = 0, o = 0
         const size_t row = ((size_t)sp * t + qrow) * a.H + h;
-        if (hh == 0 && dh == 0) *reinterpret_cast<f32x2*>(a.part_ml + 2 * row) = f32x2{m_run, l_tot};
-        float* prow = a.part_o + row * HD + dh * HDV;
+        if (hh == 0) *reinterpret_cast<f32x2*>(a.part_ml + 2 * row) = f32x2{m_run, l_tot};
+        float* prow = a.part_o + row * HD;
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
@@ -702,8 +573,8 @@ __global__ __launch_bounds__(256, HD > 128 ? 1 : 2) void attn_prefill_kernel(Pre
         return;
     }
     const float inv = 1.f / l_tot;
-    float* orow = a.out + ((size_t)qrow * a.H + h) * HD + dh * HDV;
-    const float* grow = a.gate ? a.gate + ((size_t)qrow * a.H + h) * a.gate_stride + dh * HDV : nullptr;
+    float* orow = a.out + ((size_t)qrow * a.H + h) * HD;
+    const float* grow = a.gate ? a.gate + ((size_t)qrow * a.H + h) * a.gate_stride : nullptr;
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
@@ -979,10 +850,7 @@ __global__ __launch_bounds__(256, 1) void attn_prefill_kh_kernel(PrefillArgs a) 
                     va[st] = f16x8{v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
                 }
             };
-            // Operands PVD blocks ahead: 2 at head_dim >= 256, where one wave
-            // per SIMD waits out each LDS round trip (+1.2% on Gemma's 4k
-            // prefill; 3 measured the same), 1 below.
-            constexpr int PVD = HD >= 256 ? 2 : 1;
+            constexpr int PVD = 1;  // operands one block ahead
             static_assert(PVD < NB, "operand ring");
             f16x8 va[PVD + 1][2];
 #pragma unroll
@@ -1479,46 +1347,47 @@ static bool use_ping_pong(int hd, long n_tokens, long n_heads, lmx_dtype q_dt) {
     return (n_tokens + kPpBM - 1) / kPpBM * n_heads >= 512;
 }
 
-// Query heads per prefill workgroup (they share one kv head).  At head_dim
-// 256 two heads of a kv group share a workgroup (64 rows each): a 1024-key
-// window then spans fewer key tiles per workgroup at the same MFMA work per
-// tile.  At head_dim 512 (wave pairs, two 32-row blocks a workgroup) one.
-// LMX_PREFILL_GP=1|2|4 overrides it (tuning overrides, for tests and sweeps)
-// where it divides G and the workgroup has that many row blocks.
-static int prefill_gp(int hd, int G, bool pp) {
-    const int blocks = hd >= 512 ? 2 : 4;
-    if (const int v = tuning().prefill_gp; v > 0 && G % v == 0 && v <= blocks) return v;
-    if (pp || hd >= 512) return 1;
-    return hd >= 256 && G % 2 == 0 ? 2 : 1;
+// Query heads per prefill workgroup (they share one kv head) at head_dim 64
+// and 128: one.  LMX_PREFILL_GP=1|2|4 overrides it (tuning overrides, for
+// tests and sweeps) where it divides G.
+static int prefill_gp(int G) {
+    const int v = tuning().prefill_gp;
+    return v > 0 && G % v == 0 ? v : 1;
 }
 
-// Query rows per attn_prefill_kernel workgroup and head: 32 per row block.
-static int prefill_rows(int hd, int gp) { return (hd >= 512 ? kPfBM / 2 : kPfBM) / gp; }
-
-// Key splits for attn_prefill_kernel.  When the query tiles give fewer
-// workgroups than the CUs hold at once (two per CU, one at head_dim 256), as
-// for a short chunk on a long cache, each tile's key range is cut into splits
-// until that many are in flight, keeping at least kMinSplitTiles tiles per
-// split; a merge kernel combines them.
+// Key splits for attn_prefill_kernel and attn_prefill_wide_kernel.  When the
+// query tiles give fewer workgroups than the CUs hold at once (two per CU, one
+// of the wide kernel's), as for a short chunk on a long cache, each tile's key
+// range is cut into splits until that many are in flight, keeping at least
+// kMinSplitTiles tiles of 64 keys per split (half as many in the wide kernel,
+// whose tiles cost four times the MFMAs a row); a merge kernel combines them.
 constexpr int kMinSplitTiles = 8;
 constexpr int kMaxSplits = 16;
 constexpr int kCus = 256;
 int decode_max_vis(const lmx_attn_params* p);
+// attn_prefill_wide.hip: head_dim 256 and 512
+int prefill_wide_rows(int hd);
+int prefill_wide_gp(int G);
+lmx_status prefill_wide(const PrefillArgs& a, int hd, lmx_dtype q_dt, bool lin, hipStream_t st);
+
 static int prefill_splits(const lmx_attn_params* p, lmx_dtype q_dt) {
     const int hd = (int)p->head_dim;
     if (use_ping_pong(hd, (long)p->n_tokens, (long)p->n_heads, q_dt)) return 1;
-    const int gp = prefill_gp(hd, (int)(p->n_heads / p->n_kv_heads), false);
-    const long bm = prefill_rows(hd, gp);
+    const bool wide = hd >= 256;
+    const int G = (int)(p->n_heads / p->n_kv_heads);
+    const int gp = wide ? prefill_wide_gp(G) : prefill_gp(G);
+    const long bm = wide ? prefill_wide_rows(hd) / gp : kPfBM / gp;
     const long n_wg = (long)((p->n_tokens + bm - 1) / bm) * (p->n_heads / gp);
-    const long slots = (long)kCus * (hd > 128 ? 1 : 2);
+    const long slots = (long)kCus * (wide ? 1 : 2);
     if (n_wg >= slots) return 1;
-    const int bn = hd >= 256 ? 32 : 64;
+    const int bn = 64;
     // the longest key range a workgroup covers: one query's range plus the
     // spread of the tile's positions
     const long tiles = ((long)decode_max_vis(p) + bm + bn - 1) / bn + 1;
-    long sp = (slots + n_wg - 1) / n_wg;
-    if (sp > tiles / kMinSplitTiles) sp = tiles / kMinSplitTiles;
-    if (sp > kMaxSplits) sp = kMaxSplits;
+    long sp = wide ? slots / n_wg : (slots + n_wg - 1) / n_wg;
+    const int min_tiles = wide ? kMinSplitTiles / 2 : kMinSplitTiles, max_splits = wide ? 4 * kMaxSplits : kMaxSplits;
+    if (sp > tiles / min_tiles) sp = tiles / min_tiles;
+    if (sp > max_splits) sp = max_splits;
     return sp < 2 ? 1 : (int)sp;
 }
 
@@ -1569,8 +1438,9 @@ lmx_status prefill_fwd(const lmx_attn_params* p, const AttnIo& io, const void* q
     window_magic((uint32_t)a.window, &a.w_magic, &a.w_shift);
     const int hd = (int)p->head_dim;
     const bool pp = use_ping_pong(hd, (long)p->n_tokens, (long)p->n_heads, q_dt);
-    a.gp = prefill_gp(hd, a.G, pp);
-    const int bm = pp ? kPpBM / a.gp : prefill_rows(hd, a.gp);
+    const bool wide = hd >= 256;
+    a.gp = wide ? prefill_wide_gp(a.G) : prefill_gp(a.G);
+    const int bm = wide ? prefill_wide_rows(hd) / a.gp : pp ? kPpBM / a.gp : kPfBM / a.gp;
     a.n_qtiles = (a.n_tokens + bm - 1) / bm;
     long nblk = (long)a.n_qtiles * (a.H / a.gp) * a.n_split;
     // Linear addressing: no k_cur rows and every position below the window;
@@ -1604,7 +1474,10 @@ lmx_status prefill_fwd(const lmx_attn_params* p, const AttnIo& io, const void* q
         if (lin) hipLaunchKernelGGL((attn_prefill_pp_kernel<QT, 128, true>), grid, dim3(512), 0, st, a); \
         else hipLaunchKernelGGL((attn_prefill_pp_kernel<QT, 128, false>), grid, dim3(512), 0, st, a);   \
     } while (0)
-    if (kh) {  // f16 queries only
+    if (wide) {
+        const lmx_status s = prefill_wide(a, hd, q_dt, lin, st);
+        if (s != LMX_OK) return s;
+    } else if (kh) {  // f16 queries only
         if (hd == 64) hipLaunchKernelGGL((attn_prefill_kh_kernel<f16, 64>), grid, dim3(256), 0, st, a);
         else hipLaunchKernelGGL((attn_prefill_kh_kernel<f16, 128>), grid, dim3(256), 0, st, a);
     } else if (pp) {  // f16 queries only
@@ -1612,14 +1485,10 @@ lmx_status prefill_fwd(const lmx_attn_params* p, const AttnIo& io, const void* q
     } else if (q_dt == LMX_F16) {
         if (hd == 64) LMX_PF(f16, 64);
         else if (hd == 128) LMX_PF(f16, 128);
-        else if (hd == 256) LMX_PF(f16, 256);
-        else if (hd == 512) LMX_PF(f16, 512);
         else return LMX_E_UNSUPPORTED;
     } else {
         if (hd == 64) LMX_PF(float, 64);
         else if (hd == 128) LMX_PF(float, 128);
-        else if (hd == 256) LMX_PF(float, 256);
-        else if (hd == 512) LMX_PF(float, 512);
         else return LMX_E_UNSUPPORTED;
     }
 #undef LMX_PF
