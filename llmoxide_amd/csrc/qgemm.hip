@@ -1,6 +1,6 @@
-// Quantized GEMM on gfx950 matrix cores: Y[t][r] = sum_k W[r][k] X[t][k] for
-// a batch of tokens (prefill) and a weight matrix in ggml's on-disk block
-// formats Q4_K, Q6_K or Q8_0, read once per launch.
+// GEMM on gfx950 matrix cores: Y[t][r] = sum_k W[r][k] X[t][k] for a batch of
+// tokens and a weight matrix in ggml's on-disk formats Q4_K, Q6_K, Q8_0, F16
+// or BF16, read once per launch.
 //
 // Replaces the reference's prefill GEMM (gemm_q6k in gemm.wgsl:93-95 and
 // gemm_q6k.metal:50, chosen from 16 tokens: crates/gpu/src/lib.rs:1039-1046,
@@ -12,94 +12,98 @@
 //     Q4_K  q in [0, 15],     s = d * sc_g, o = -dmin * m_g  (groups of 32)
 //     Q6_K  q in [-32, 31],   s = d * sc_g, o = 0            (groups of 16)
 //     Q8_0  q in [-128, 127], s = d,        o = 0            (groups of 32)
-//   so   y = sum_g  s_g * (sum_{k in g} q_k x_k)  +  o_g * (sum_{k in g} x_k),
-//   the order dot_row itself uses for Q4_K (its s1 and x1 per sub-block).
-//   The integers q are exact in f16; x is split into f16 x_hi + x_lo
-//   (|x - x_hi - x_lo| <= 2^-22 |x|), so each group's integer sum is two
-//   v_mfma_f32_32x32x16_f16 products accumulated in fp32, and the group's
-//   scale and offset are applied in fp32 (the x sums come from the fp32 x).
+//   x is split into f16 x_hi + x_lo (|x - x_hi - x_lo| <= 2^-22 |x|), and all
+//   products run on v_mfma_f32_32x32x16_f16 with fp32 accumulation.  The
+//   integer scales go into the weight operand, where the vector unit pays for
+//   them once a weight instead of once a token: sc_g q of Q4_K is at most 945
+//   and exact in f16; of Q6_K it is at most 4096 and exact as f16(sc_g q) plus
+//   a remainder (third product: remainder times x_hi).  Only d, one a
+//   super-block of 256, is applied to the fp32 sums (of a bf16 row, the power
+//   of two that brought 256 / KQ of its weights into f16's range).  Q4_K's offsets are one
+//   more MFMA a super-block: the m_g against the group sums of x (hi and lo,
+//   scaled by 1/16 into f16's range).  Q8_0's d has 11 bits of its own, so its
+//   group sums are scaled in fp32.
 //
 //   Range: before the split, each token's x is multiplied by a power of two
 //   2^k_t (exact).  k_t is the running minimum over the chunks of a bound
 //   k_c: 0 while the token's largest |x| in the chunk lies in [2^-6, 2^14),
-//   else the k that brings it into [2^14, 2^15).  So no scaled value comes
+//   else the k that brings it into [2^13, 2^14).  So no scaled value comes
 //   near f16's 65504, and a token whose x are all tiny is scaled up instead
 //   of falling into f16 subnormals.  Every partial sum of a token is in one
-//   scaled domain: when a chunk changes k_t, the token's accumulated y is
+//   scaled domain: when a chunk lowers k_t, the token's accumulated y is
 //   first multiplied by the (exact) ratio, and the store multiplies by
 //   2^-k_t.  Elements far below their chunk's maximum keep an absolute error
-//   of about 2^-22 of the largest value met, as fp32 summation would.  In
-//   the common case (k_t = 0 from the first chunk on) the scaling is skipped.
+//   of about 2^-22 of the largest value met, as fp32 summation would.
 //
-// Tiles.  A workgroup owns 64 tokens x 128 weight rows.  Its four consumer
-// waves multiply: wave (wm, wn) owns tokens 32 wm .. + 31 and rows
-// 64 wn .. + 63, two 32 x 32 MFMA tiles with x as the A operand and q as B,
-// so each lane of a result tile holds one weight row and 16 tokens, and a
-// group's scale is one value per lane.  K goes through LDS 128 weights at a
-// time (half a K-quant super-block, four Q8_0 blocks): x as swizzled f16 hi /
-// lo rows, W decoded to f16 integers with each row's group scales, and the
-// (token, group) x sums.  Its producer waves, four or eight for W (load and
-// decode) and four for x (load, hi / lo split and group sums), stash the next chunk
-// into the other of two LDS buffers meanwhile, with the chunk after that
-// already in registers.
+// A workgroup of eight waves owns 32 TT tokens x 32 RT WR rows and walks K in
+// chunks of 256.  x goes through LDS, two buffers of swizzled f16 hi / lo
+// rows: each wave loads, splits and stores TM / 8 tokens of the next chunk
+// beside its MFMAs, its loads a chunk ahead of that.  A chunk's raw weight
+// bytes come from memory straight to LDS, in 16-byte pieces that cover each
+// row's block (whole lines; 2- and 4-byte loads of the 2-byte aligned fields
+// kept the address unit busy for longer than the MFMAs); each wave reads the
+// bytes of its own k range (KQ = 8 / WR ranges a chunk) into registers, and
+// decodes them there into MFMA operands, each weight once a workgroup.  The
+// KQ partial sums meet in LDS at the end.
+//
+// Measured (in_dim 4096, us a call; before: 64 x 128 tiles with one wave kind
+// per stage for the block formats, four tokens a launch for dense rows):
+// 16 tokens x 4096 rows Q4_K 81 -> 26, Q6_K 116 -> 29, Q8_0 94 -> 23, bf16
+// 103 -> 26; 500 x 1024 rows 83 -> 40, 120 -> 38, 99 -> 34, 2577 -> 37; 64 x
+// 4096 rows bf16 433 -> 37.  What bounds it: a chunk's round trip (its x and W
+// loads are a chunk ahead, about 1.5 us) and x's staging (1.2 us of vector
+// work a chunk at 64 tokens), against 0.3 us of MFMAs at 64 x 32.
+#include <algorithm>
+#include <climits>
+
 #include "common.hpp"
+#include "lds_dma.hpp"
 
 namespace lmx {
 
-enum GType { kGQ8_0 = 8, kGQ4K = 12, kGQ6K = 14 };
-
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-#ifndef LMX_QGEMM_ROWS
-#define LMX_QGEMM_ROWS 128
-#endif
-constexpr int kGM = 64;        // tokens per workgroup
-constexpr int kGN = LMX_QGEMM_ROWS;  // weight rows per workgroup (64 or 128)
-#ifndef LMX_QGEMM_CONS
-#define LMX_QGEMM_CONS 4
-#endif
-constexpr int kGCons = LMX_QGEMM_CONS;         // consumer (MFMA) waves: 4 or 8
-constexpr int kNTW = kGN / (16 * kGCons);      // 32-row MFMA tiles per consumer wave
-constexpr int kGK = 128;       // weights per LDS chunk
-constexpr int kGXF = 2048;                       // float4s of x in a chunk (64 tokens x 128)
-constexpr int kGConsT = 64 * kGCons;             // consumer threads
-// W-producer threads per row: 4 for Q6_K (one 32-weight unit each: its
-// decode is the heaviest), 2 for Q4_K and Q8_0 (two units each; 4 measured
-// 2% slower for them).
+enum GType { kGF16 = 1, kGQ8_0 = 8, kGQ4K = 12, kGQ6K = 14, kGBF16 = 30 };
 template <int TY>
-constexpr int g_wparts() { return TY == kGQ6K ? 4 : 2; }
-// x-producer threads: 512 (four float4s of a chunk each) for Q4_K, whose x
-// producers also form the group sums (73 -> 63.5 us against 256), 256 (eight
-// each) for Q8_0 (512 measured 5% slower) and Q6_K (eight W waves).
-template <int TY>
-constexpr int g_xthreads() { return TY == kGQ4K ? 512 : 256; }
-template <int TY>
-constexpr int g_threads() { return kGConsT + kGN * g_wparts<TY>() + g_xthreads<TY>(); }  // consumers, W, x producers
+constexpr bool g_dense() { return TY == kGF16 || TY == kGBF16; }
 
+constexpr int kGK = 256;  // k per chunk: a K-quant super-block, eight Q8_0 blocks
+
+// Bytes of a chunk of a row, the 16-byte pieces that cover it at its largest
+// misalignment (blocks of Q4_K are 16-byte aligned, the others 2-byte), and
+// the pieces' stride in LDS: odd, so that 16 rows of one piece meet all banks.
 template <int TY>
 struct GTraits;
-template <> struct GTraits<kGQ4K> { static constexpr int gs = 32, words = 12; };
-template <> struct GTraits<kGQ6K> { static constexpr int gs = 16, words = 9; };
-template <> struct GTraits<kGQ8_0> { static constexpr int gs = 32, words = 9; };
+template <> struct GTraits<kGQ4K> { static constexpr int bytes = 144, pieces = 9, stride = 9; };
+template <> struct GTraits<kGQ6K> { static constexpr int bytes = 210, pieces = 14, stride = 15; };
+template <> struct GTraits<kGQ8_0> { static constexpr int bytes = 272, pieces = 18, stride = 19; };
+template <> struct GTraits<kGF16> { static constexpr int bytes = 512, pieces = 32, stride = 33; };
+template <> struct GTraits<kGBF16> { static constexpr int bytes = 512, pieces = 32, stride = 33; };
 
 struct GemmArgs {
     const uint8_t* w;
     const float* x;
     float* y;
     int rows, in_dim, n_tok;
-    size_t row_bytes;
+    size_t row_bytes, w_bytes;
 };
 
-// Largest x over each group of 32 lanes (x >= 0): DPP within each 16-lane
-// row, then one swizzle between the two rows of a group (no LDS traffic,
-// unlike ds_bpermute).
-__device__ __forceinline__ float max32(float x) {
+// max(|a|, |b|, c) as one instruction (fmaxf first quiets each operand).
+__device__ __forceinline__ float absmax3(float a, float b, float c) {
+    float r;
+    asm("v_max3_f32 %0, |%1|, |%2|, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+// Largest x over the wave's 64 lanes (x >= 0).
+__device__ __forceinline__ float wave_max64(float x) {
     x = fmaxf(x, dpp<0xB1>(x));   // quad_perm [1,0,3,2]
     x = fmaxf(x, dpp<0x4E>(x));   // quad_perm [2,3,0,1]
     x = fmaxf(x, dpp<0x141>(x));  // row_half_mirror
     x = fmaxf(x, dpp<0x140>(x));  // row_mirror
-    // swizzle, bitmask mode: lane ^ 16 within 32
-    return fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, x), 0x401F)));
+    const int b = __builtin_bit_cast(int, x);
+    const float r0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 0));
+    const float r1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 16));
+    const float r2 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 32));
+    const float r3 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 48));
+    return fmaxf(fmaxf(r0, r1), fmaxf(r2, r3));
 }
 // Sum over each aligned group of 8 lanes; every lane of the group gets it.
 __device__ __forceinline__ float sum8(float x) {
@@ -108,442 +112,547 @@ __device__ __forceinline__ float sum8(float x) {
     return x + dpp<0x141>(x);  // row_half_mirror: lane i with 7 - i of its 8
 }
 
-// Swizzled offset (in halfs) of 8-half chunk c of LDS row r: the chunk index
-// is XORed with the row, so the rows an MFMA operand read touches spread
-// over the banks.
-__device__ __forceinline__ int sw(int r, int c) { return r * kGK + ((c ^ (r & 15)) << 3); }
-
-// Eight bytes at a 2-byte aligned address as two dwords: the covering
-// aligned dwords, funnel-shifted.  A shifted read also touches the 2 bytes
-// after the range; every range below ends at least 2 bytes before its block.
-__device__ __forceinline__ void ld8_a2(const uint8_t* p, uint32_t* o) {
-    const uint32_t sh = (uint32_t)(reinterpret_cast<uintptr_t>(p) & 3);
+__device__ __forceinline__ f16x2 as_h2(uint32_t x) { return __builtin_bit_cast(f16x2, x); }
+__device__ __forceinline__ uint32_t lds_u16(const uint8_t* p) { return *reinterpret_cast<const uint16_t*>(p); }
+// N dwords at a 2-byte aligned LDS address.
+template <int N>
+__device__ __forceinline__ void lds_words(const uint8_t* p, uint32_t (&o)[N]) {
+    const uint32_t sh = (uint32_t)(reinterpret_cast<uintptr_t>(p) & 2);
     const uint32_t* b = reinterpret_cast<const uint32_t*>(p - sh);
-    const uint32_t r0 = b[0], r1 = b[1], r2 = sh ? b[2] : 0u;
-    o[0] = __builtin_amdgcn_alignbyte(r1, r0, sh);
-    o[1] = __builtin_amdgcn_alignbyte(r2, r1, sh);
-}
-
-__device__ __forceinline__ float half_bits(uint32_t h) {
-    return (float)__builtin_bit_cast(f16, (uint16_t)(h & 0xFFFF));
-}
-__device__ __forceinline__ uint32_t byte_of(const uint32_t* w, int i) { return (w[i >> 2] >> (8 * (i & 3))) & 0xFF; }
-
-// Raw W bytes of one 32-weight unit (row, part) of a chunk: four units a
-// row, each 32 of the chunk's 128 weights.
-//  Q4_K: chunk = half hf of a super-block; part p is sub-block 4 hf + p, one
-//        nibble (p & 1) of the 32 quant bytes of pair 2 hf + (p >> 1):
-//        words 0-3 the block header (d, dmin, 12 scale bytes), 4-11 the
-//        pair's quant bytes.
-//  Q6_K: chunk = half h; part p takes l in [8 p, 8 p + 8) of every 32-wide
-//        quarter: words 0-1 ql[8 p ..], 2-3 ql[32 + 8 p ..], 4-5 qh[8 p ..]
-//        (of the half), 6-7 the half's 8 scales, 8 d.
-//  Q8_0: chunk = four blocks; part p takes block p (34 bytes: words 0-7
-//        bytes 0-31 from a 2-byte aligned start, word 8 bytes 32-33).
-template <int TY>
-__device__ __forceinline__ void load_w(const uint8_t* row, int k0, int part, uint32_t* rw) {
-    if constexpr (TY == kGQ4K) {
-        const uint8_t* blk = row + (size_t)(k0 >> 8) * 144;
-        const int hf = (k0 >> 7) & 1;
-        const u32x4 h4 = *reinterpret_cast<const u32x4*>(blk);
-        const uint8_t* qb = blk + 16 + 32 * (2 * hf + (part >> 1));
-        const u32x4 q0 = *reinterpret_cast<const u32x4*>(qb);
-        const u32x4 q1 = *reinterpret_cast<const u32x4*>(qb + 16);
+    uint32_t raw[N + 1];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            rw[i] = h4[i];
-            rw[4 + i] = q0[i];
-            rw[8 + i] = q1[i];
-        }
-    } else if constexpr (TY == kGQ6K) {
-        const uint8_t* blk = row + (size_t)(k0 >> 8) * 210;
-        const int h = (k0 >> 7) & 1;
-        const uint8_t* ql = blk + 64 * h + 8 * part;
-        ld8_a2(ql, rw + 0);
-        ld8_a2(ql + 32, rw + 2);
-        ld8_a2(blk + 128 + 32 * h + 8 * part, rw + 4);
-        ld8_a2(blk + 192 + 8 * h, rw + 6);
-        rw[8] = *reinterpret_cast<const uint16_t*>(blk + 208);
-    } else {
-        const uint8_t* blk = row + (size_t)((k0 >> 5) + part) * 34;
+    for (int i = 0; i <= N; ++i) raw[i] = b[i];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) ld8_a2(blk + 8 * i, rw + 2 * i);
-        rw[8] = *reinterpret_cast<const uint16_t*>(blk + 32);
+    for (int i = 0; i < N; ++i) o[i] = __builtin_amdgcn_alignbyte(raw[i + 1], raw[i], sh);
+}
+// Four small unsigned integers (bytes) as f16 + 1024, in the order 0 2 1 3 in
+// which x is stored (masks instead of byte moves).
+__device__ __forceinline__ void bytes_1024(uint32_t q, f16x2& a, f16x2& b) {
+    a = as_h2((q & 0x00FF00FFu) | 0x64006400u);
+    b = as_h2(((q >> 8) & 0x00FF00FFu) | 0x64006400u);
+}
+__device__ __forceinline__ f16x2 pk_fma(f16x2 a, f16x2 b, f16x2 c) { return __builtin_elementwise_fma(a, b, c); }
+
+// A wave's share of a chunk of one weight row: its raw bytes, read from LDS
+// once, and the operand of each of its k-steps.  KQ ranges a chunk; lane half
+// hh holds 8 weights a step.
+//   Q4_K  range = pair of sub-blocks (KQ 4) or one (KQ 8); the half's 16 quant
+//         bytes; steps: low nibbles of bytes 0-7, 8-15, then the high ones
+//   Q6_K  range = half h, l in [16 lq, + 16) of every quarter k (KQ 4) or of
+//         quarters 2 kn, 2 kn + 1 (KQ 8); the half's 8 l; a step per quarter,
+//         which is one scale group
+//   Q8_0  range = two blocks (KQ 4) or one; the half's 16 weights of each
+template <int TY, int KQ>
+struct WFrag;
+
+template <int KQ>
+struct WFrag<kGQ4K, KQ> {
+    static constexpr int NK = 16 / KQ;
+    uint32_t hdr[4], q[4];
+    __device__ __forceinline__ void load(const uint8_t* blk, int kq, int hh) {
+        const uint4 h = *reinterpret_cast<const uint4*>(blk);
+        const uint4 v = *reinterpret_cast<const uint4*>(blk + 16 + 32 * (KQ == 4 ? kq : kq >> 1) + 16 * hh);
+        hdr[0] = h.x; hdr[1] = h.y; hdr[2] = h.z; hdr[3] = h.w;
+        q[0] = v.x; q[1] = v.y; q[2] = v.z; q[3] = v.w;
     }
-}
-
-// Eight small integers as f16 into 8-half chunk c of LDS row r.
-__device__ __forceinline__ void put8(f16* q_s, int r, int c, const int (&v)[8]) {
-    f16x8 h;
+    __device__ static __forceinline__ int k_of(int s, int kq, int hh) {
+        return KQ == 4 ? 64 * kq + 32 * (s >> 1) + 16 * hh + 8 * (s & 1) : 32 * kq + 16 * hh + 8 * s;
+    }
+    // 6-bit scale and min of sub-block j, quant.rs:33-47
+    __device__ __forceinline__ uint32_t scale(int j) const {
+        const int s = 8 * (j & 3);
+        const uint32_t b0 = (hdr[1] >> s) & 0xFF, b2 = (hdr[3] >> s) & 0xFF;
+        return j < 4 ? b0 & 63 : (b2 & 0xF) | ((b0 >> 6) << 4);
+    }
+    __device__ __forceinline__ f16x8 step(int s, int kq) const {
+        const int j = KQ == 4 ? 2 * kq + (s >> 1) : kq;  // sub-block
+        const int hi = 4 * (j & 1);
+        const f16 sc = (f16)(float)scale(j);
+        const f16x2 s2 = {sc, sc}, n2 = f16x2{(f16)-1024.f, (f16)-1024.f} * s2;
+        f16x8 o;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) h[j] = (f16)(float)v[j];
-    *reinterpret_cast<f16x8*>(&q_s[sw(r, c)]) = h;
-}
-
-// Decode thread (row r, part)'s raw bytes into q_s (f16 integers) and its
-// groups' (scale, offset) into so_s.
-template <int TY>
-__device__ __forceinline__ void stash_w(const uint32_t* rw, int k0, int r, int part, bool live, f16* q_s,
-                                        f32x2* so_s) {
-    constexpr int NG = kGK / GTraits<TY>::gs;
-    if constexpr (TY == kGQ4K) {
-        // weights 32 part + e of the chunk: nibble (part & 1) of quant byte e
-        // of the pair (quant.rs:54-128)
-        const uint32_t* q = rw + 4;
-        const int nib = 4 * (part & 1);
-#pragma unroll
-        for (int cc = 0; cc < 4; ++cc) {
-            int v[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = (int)((byte_of(q, 8 * cc + j) >> nib) & 0xF);
-            put8(q_s, r, 4 * part + cc, v);
+        for (int i = 0; i < 2; ++i) {
+            const uint32_t v = q[2 * (s & 1) + i] >> hi;
+            // (1024 + q) sc - 1024 sc, exact
+            const f16x2 a = pk_fma(as_h2((v & 0x000F000Fu) | 0x64006400u), s2, n2);
+            const f16x2 b = pk_fma(as_h2(((v >> 8) & 0x000F000Fu) | 0x64006400u), s2, n2);
+            o[4 * i] = a[0]; o[4 * i + 1] = a[1]; o[4 * i + 2] = b[0]; o[4 * i + 3] = b[1];
         }
-        // sub-block j = 4 hf + part: scale and min, quant.rs:33-47
-        const int j = 4 * ((k0 >> 7) & 1) + part;
-        const float d = half_bits(rw[0]), dmin = half_bits(rw[0] >> 16);
-        const uint32_t* sc6 = rw + 1;  // the 12 scale bytes
-        uint32_t sc, m;
-        if (j < 4) {
-            sc = byte_of(sc6, j) & 63;
-            m = byte_of(sc6, j + 4) & 63;
-        } else {
-            sc = (byte_of(sc6, j + 4) & 0xF) | ((byte_of(sc6, j - 4) >> 6) << 4);
-            m = (byte_of(sc6, j + 4) >> 4) | ((byte_of(sc6, j) >> 6) << 4);
+        return o;
+    }
+    __device__ __forceinline__ float d() const { return (float)as_h2(hdr[0])[0]; }
+    __device__ __forceinline__ float dmin() const { return (float)as_h2(hdr[0])[1]; }
+    __device__ __forceinline__ f16x8 mins() const {
+        f16x8 m;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t b1 = (hdr[2] >> (8 * j)) & 0xFF, b2 = (hdr[3] >> (8 * j)) & 0xFF;
+            m[j] = (f16)(float)(b1 & 63);
+            m[j + 4] = (f16)(float)((b2 >> 4) | ((b1 >> 6) << 4));
         }
-        so_s[r * NG + part] = live ? f32x2{d * (float)sc, -(dmin * (float)m)} : f32x2{0.f, 0.f};
-    } else if constexpr (TY == kGQ6K) {
-        // weight 32 k + l of the half (l = 8 part + j): low / high nibble
-        // (k >> 1) of ql[l + 32 (k & 1)], with bits 2k, 2k + 1 of qh[l] on
-        // top, minus 32
+        return m;
+    }
+};
+
+template <int KQ>
+struct WFrag<kGQ6K, KQ> {
+    static constexpr int NK = 16 / KQ;
+    uint32_t la[2], lb[2], h[2], sc[2], dd;
+    __device__ __forceinline__ void load(const uint8_t* blk, int kq, int hh) {
+        const int half = KQ == 4 ? kq >> 1 : kq >> 2, lq = KQ == 4 ? kq & 1 : (kq >> 1) & 1;
+        const int l0 = 16 * lq + 8 * hh;
+        lds_words<2>(blk + 64 * half + l0, la);
+        lds_words<2>(blk + 64 * half + 32 + l0, lb);
+        lds_words<2>(blk + 128 + 32 * half + l0, h);
+        lds_words<2>(blk + 192 + 8 * half, sc);
+        dd = lds_u16(blk + 208);
+    }
+    __device__ static __forceinline__ int quarter(int s, int kq) { return KQ == 4 ? s : 2 * (kq & 1) + s; }
+    __device__ static __forceinline__ int k_of(int s, int kq, int hh) {
+        const int half = KQ == 4 ? kq >> 1 : kq >> 2, lq = KQ == 4 ? kq & 1 : (kq >> 1) & 1;
+        return 128 * half + 32 * quarter(s, kq) + 16 * lq + 8 * hh;
+    }
+    // hi + lo = sc q, both exact
+    __device__ __forceinline__ void step(int s, int kq, f16x8& hi, f16x8& lo) const {
+        const int k = quarter(s, kq), lq = KQ == 4 ? kq & 1 : (kq >> 1) & 1;
+        const int g = 2 * k + lq;
+        const f16 c = (f16)(float)(int8_t)((g < 4 ? sc[0] : sc[1]) >> (8 * (g & 3)));
+        const f16x2 c2 = {c, c}, off = {(f16)-1056.f, (f16)-1056.f};
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            int v[8];
+        for (int i = 0; i < 2; ++i) {
+            const uint32_t ql = ((k & 1) ? lb[i] : la[i]) >> (4 * (k >> 1));
+            const uint32_t q = (ql & 0x0F0F0F0Fu) | (((h[i] >> (2 * k)) << 4) & 0x30303030u);
+            f16x2 a, b;
+            bytes_1024(q, a, b);
+            a += off;
+            b += off;
+            const f16x2 ah = a * c2, bh = b * c2;
+            const f16x2 al = pk_fma(a, c2, -ah), bl = pk_fma(b, c2, -bh);
+            hi[4 * i] = ah[0]; hi[4 * i + 1] = ah[1]; hi[4 * i + 2] = bh[0]; hi[4 * i + 3] = bh[1];
+            lo[4 * i] = al[0]; lo[4 * i + 1] = al[1]; lo[4 * i + 2] = bl[0]; lo[4 * i + 3] = bl[1];
+        }
+    }
+    __device__ __forceinline__ float d() const { return (float)as_h2(dd)[0]; }
+};
+
+template <int KQ>
+struct WFrag<kGQ8_0, KQ> {
+    static constexpr int NK = 16 / KQ, NB = NK / 2;
+    uint32_t q[NB][4], dd[NB];
+    __device__ __forceinline__ void load(const uint8_t* blk, int kq, int hh) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const uint32_t lb = byte_of(rw + 2 * (k & 1), j);
-                const uint32_t hb = byte_of(rw + 4, j);
-                v[j] = (int)(((lb >> (4 * (k >> 1))) & 0xF) | (((hb >> (2 * k)) & 3) << 4)) - 32;
+        for (int b = 0; b < NB; ++b) {
+            const uint8_t* p = blk + 34 * (NB * kq + b);
+            dd[b] = lds_u16(p);
+            lds_words<4>(p + 2 + 16 * hh, q[b]);
+        }
+    }
+    __device__ static __forceinline__ int k_of(int s, int kq, int hh) {
+        return 32 * (NB * kq + (s >> 1)) + 16 * hh + 8 * (s & 1);
+    }
+    __device__ __forceinline__ f16x8 step(int s) const {
+        const f16x2 off = {(f16)-1152.f, (f16)-1152.f};
+        f16x8 o;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            f16x2 a, b;
+            bytes_1024(q[s >> 1][2 * (s & 1) + i] ^ 0x80808080u, a, b);  // q + 128
+            a += off;
+            b += off;
+            o[4 * i] = a[0]; o[4 * i + 1] = a[1]; o[4 * i + 2] = b[0]; o[4 * i + 3] = b[1];
+        }
+        return o;
+    }
+    __device__ __forceinline__ float d(int b) const { return (float)as_h2(dd[b])[0]; }
+};
+
+// Dense rows: range = 256 / KQ consecutive weights.  bf16 becomes f16 times a
+// power of two that brings the range's largest weight into [2^14, 2^15): exact
+// for weights down to 2^-31 of it, 2^-39 of it below.
+template <int TY, int KQ>
+struct DFrag {
+    static constexpr int NK = 16 / KQ;
+    uint4 raw[NK];
+    int sc;
+    __device__ static __forceinline__ int k_of(int s, int kq, int hh) { return 16 * (NK * kq + s) + 8 * hh; }
+    // left: weights of the chunk that lie inside the row
+    __device__ __forceinline__ void load(const uint8_t* row, int kq, int hh, int left) {
+        uint32_t top = 0;
+#pragma unroll
+        for (int s = 0; s < NK; ++s) {
+            const int k = k_of(s, kq, hh);
+            raw[s] = k < left ? *reinterpret_cast<const uint4*>(row + 2 * k) : uint4{0u, 0u, 0u, 0u};
+            if constexpr (TY == kGBF16) {
+                const uint32_t w[4] = {raw[s].x, raw[s].y, raw[s].z, raw[s].w};
+#pragma unroll
+                for (int i = 0; i < 4; ++i) top = max(top, max(w[i] & 0x7FFF0000u, (w[i] << 16) & 0x7FFF0000u));
             }
-            put8(q_s, r, 4 * k + part, v);
         }
-        // groups of 16: g = 2 k + (l >= 16), written by parts 0 and 2
-        if ((part & 1) == 0) {
-            const float d = half_bits(rw[8]);
+        sc = 0;
+        if constexpr (TY == kGBF16) {
+            const float t = __builtin_bit_cast(float, top);
+            const float m = fmaxf(t, shfl_xor(t, 32));  // (every bit pattern orders as its float)
+            if (m > 0.f && m <= 3.402823466e38f) sc = 15 - __builtin_amdgcn_frexp_expf(m);
+        }
+    }
+    __device__ __forceinline__ f16x8 step(int s) const {
+        const uint32_t w[4] = {raw[s].x, raw[s].y, raw[s].z, raw[s].w};
+        f16x8 o;
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const int g = 2 * k + (part >> 1);
-                const float sc = (float)(int8_t)byte_of(rw + 6, g);
-                so_s[r * NG + g] = live ? f32x2{d * sc, 0.f} : f32x2{0.f, 0.f};
+        for (int i = 0; i < 4; ++i) {  // pairs (0 1) (2 3) .. into the order 0 2 1 3
+            f16 a, b;
+            if constexpr (TY == kGBF16) {
+                a = (f16)__builtin_amdgcn_ldexpf(__builtin_bit_cast(float, w[i] << 16), sc);
+                b = (f16)__builtin_amdgcn_ldexpf(__builtin_bit_cast(float, w[i] & 0xFFFF0000u), sc);
+            } else {
+                a = as_h2(w[i])[0];
+                b = as_h2(w[i])[1];
             }
+            o[4 * (i >> 1) + (i & 1)] = a;
+            o[4 * (i >> 1) + 2 + (i & 1)] = b;
         }
-    } else {
-        // block part: d at bytes 0-1, quants at bytes 2-33
-        const float d = half_bits(byte_of(rw, 0) | (byte_of(rw, 1) << 8));
-#pragma unroll
-        for (int cc = 0; cc < 4; ++cc) {
-            int v[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = (int)(int8_t)byte_of(rw, 2 + 8 * cc + j);
-            put8(q_s, r, 4 * part + cc, v);
-        }
-        so_s[r * NG + part] = live ? f32x2{d, 0.f} : f32x2{0.f, 0.f};
+        return o;
     }
-}
+    __device__ __forceinline__ float d() const { return __builtin_amdgcn_ldexpf(1.f, -sc); }
+};
+template <int KQ>
+struct WFrag<kGF16, KQ> : DFrag<kGF16, KQ> {};
+template <int KQ>
+struct WFrag<kGBF16, KQ> : DFrag<kGBF16, KQ> {};
 
-// Q8_0, two units a thread: blocks 2 pair and 2 pair + 1 of the chunk, 68
-// contiguous bytes (dword-aligned when rows are, as 4096-wide ones are) as
-// 17 words; separate 34-byte units would put every other block 2 bytes off a
-// dword (15-20% slower).
-__device__ __forceinline__ void load_q8_pair(const uint8_t* row, int k0, int pair, uint32_t* rw) {
-    const uint8_t* blk = row + (size_t)((k0 >> 5) + 2 * pair) * 34;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) ld8_a2(blk + 8 * i, rw + 2 * i);
-    // the last 4 bytes (block 2 pair + 1's final quants) as two 2-byte loads
-    rw[16] = (uint32_t)reinterpret_cast<const uint16_t*>(blk + 64)[0] |
-             ((uint32_t)reinterpret_cast<const uint16_t*>(blk + 66)[0] << 16);
-    rw[17] = 0u;
-}
-__device__ __forceinline__ void stash_q8_pair(const uint32_t* rw, int r, int pair, bool live, f16* q_s,
-                                              f32x2* so_s) {
-    constexpr int NG = kGK / GTraits<kGQ8_0>::gs;
-#pragma unroll
-    for (int bi = 0; bi < 2; ++bi) {
-        // block 2 pair + bi: d at bytes 34 bi, quants at 34 bi + 2
-        const int base = 34 * bi;
-        const float d = half_bits(byte_of(rw, base) | (byte_of(rw, base + 1) << 8));
-#pragma unroll
-        for (int cc = 0; cc < 4; ++cc) {
-            int v[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = (int)(int8_t)byte_of(rw, base + 2 + 8 * cc + j);
-            put8(q_s, r, 4 * (2 * pair + bi) + cc, v);
-        }
-        so_s[r * NG + 2 * pair + bi] = live ? f32x2{d, 0.f} : f32x2{0.f, 0.f};
-    }
-}
+template <int TY, int TT, int RT, int WR>
+__global__ __launch_bounds__(512, 1) void qgemm_kernel(GemmArgs a) {
+    constexpr int TM = 32 * TT, TN = 32 * RT * WR, KQ = 8 / WR;
+    constexpr int NK = 16 / KQ;  // k-steps of a wave per chunk
+    constexpr int STR = GTraits<TY>::stride * 16, PC = GTraits<TY>::stride, NPC = GTraits<TY>::pieces;
+    constexpr int NX = TM / 8;   // tokens a wave stages per chunk
+    constexpr bool OFFSET = TY == kGQ4K;
+    // x rows of 256 halfs, 16-byte pieces XORed with the row; also the
+    // partial sums at the end
+    constexpr int XB = TM * kGK;
+    constexpr int SMEM_X = 2 * 2 * XB * 2, SMEM_Y = KQ * TM * TN * 4;
+    __shared__ __attribute__((aligned(16))) unsigned char xy_s[SMEM_X > SMEM_Y ? SMEM_X : SMEM_Y];
+    __shared__ __attribute__((aligned(16))) unsigned char w_s[TN * STR + 16];
+    __shared__ __attribute__((aligned(16))) f16 xs_s[2][OFFSET ? TM * 16 : 8];  // x sums / 16: 8 hi, 8 lo
+    __shared__ __attribute__((aligned(16))) float rs_s[2][TM];  // a token's scale ratio of this chunk
+    __shared__ __attribute__((aligned(16))) int chg_s[2][8];    // per staging wave: some ratio is not 1
+    auto xh = [&](int b) { return reinterpret_cast<f16*>(xy_s) + b * 2 * XB; };
+    auto xl = [&](int b) { return xh(b) + XB; };
 
-template <int TY>
-__global__ __launch_bounds__(g_threads<TY>(), 1) void qgemm_kernel(GemmArgs a) {
-    constexpr int GS = GTraits<TY>::gs;
-    constexpr int NG = kGK / GS;          // groups per chunk
-    constexpr int KPG = GS / 16;          // MFMA k-steps per group
-    constexpr bool OFFSET = TY == kGQ4K;  // groups carry an offset (Q4_K's min)
-    constexpr int WW = GTraits<TY>::words;
-    // Two buffers of every stage: chunk ch lives in buffer ch & 1.
-    __shared__ __attribute__((aligned(16))) f16 xh_s[2][kGM * kGK];
-    __shared__ __attribute__((aligned(16))) f16 xl_s[2][kGM * kGK];
-    __shared__ __attribute__((aligned(16))) f16 q_s[2][kGN * kGK];
-    __shared__ __attribute__((aligned(16))) f32x2 so_s[2][kGN * NG];        // (s, o) per row, group
-    __shared__ __attribute__((aligned(16))) float xs_s[2][OFFSET ? NG * kGM : 4];  // x sums per group, token
-    // Per token: the ratio 2^(k_new - k_old) of its x scale in this chunk,
-    // and 2^-k_new.
-    __shared__ __attribute__((aligned(16))) float rs_s[2][kGM];
-    __shared__ __attribute__((aligned(16))) float iv_s[2][kGM];
-
-    const int n_tb = (a.n_tok + kGM - 1) / kGM;
+    const int n_tb = (a.n_tok + TM - 1) / TM;
     const int tb = blockIdx.x % n_tb, rb = blockIdx.x / n_tb;
-    const int t0 = tb * kGM, r0 = rb * kGN;
-    const int tid = threadIdx.x;
-    const int n_chunks = a.in_dim / kGK;
-
-    // The W-producer waves (eight for Q6_K, else four) and x-producer waves
-    // (four) load, decode and stash chunk ch + 1 while the consumer waves (the
-    // first kGCons) multiply chunk
-    // ch: a SIMD holds waves of every kind, so the producers' VALU work issues
-    // beside the consumers' MFMAs.  One barrier per chunk; every wave executes
-    // the same number of barriers.
-    constexpr int WPARTS = g_wparts<TY>(), WU = 4 / WPARTS;  // threads a row, units a thread
-    constexpr int WT = kGN * WPARTS;                           // W-producer threads
-    if (tid >= kGConsT) {
-        const bool x_prod = tid >= kGConsT + WT;  // wave-uniform
-        const int ptid = x_prod ? tid - kGConsT - WT : tid - kGConsT;
-        // ---- register prefetch of one chunk
-        // x: 64 tokens x 128 floats = 2048 float4, XU per thread; 32
-        // consecutive threads read one token's 512 contiguous bytes.
-        constexpr int XT = g_xthreads<TY>(), XU = kGXF / XT;  // x-producer threads, float4s a thread
-        f32x4 rx[XU];
-        // Running scale exponent k_t of each of this thread's tokens (100:
-        // no nonzero x seen yet; any ratio applied to a zero y is exact).
-        int kx[XU];
-#pragma unroll
-        for (int u = 0; u < XU; ++u) kx[u] = 100;
-        bool ones[2] = {false, false};  // buffer b holds (1, 1) for this wave's tokens (wave-uniform)
-        constexpr bool Q8PAIR = TY == kGQ8_0 && WU == 2;
-        uint32_t rw[WU][Q8PAIR ? 18 : WW];
-        const int w_row = ptid / WPARTS, w_part = ptid % WPARTS;
-        const bool w_thread = w_row < kGN;  // threads past the tile's rows stage no W
-        const bool w_live = w_thread && r0 + w_row < a.rows;
-        const uint8_t* wrow = a.w + (size_t)(w_live ? r0 + w_row : 0) * a.row_bytes;
-        auto load_chunk = [&](int k0) {
-            if (x_prod) {
-#pragma unroll
-                for (int u = 0; u < XU; ++u) {
-                    const int i = ptid + XT * u, tok = i >> 5, k4 = i & 31;
-                    f32x4 v = {0.f, 0.f, 0.f, 0.f};
-                    if (t0 + tok < a.n_tok)
-                        v = *reinterpret_cast<const f32x4*>(a.x + (size_t)(t0 + tok) * a.in_dim + k0 + 4 * k4);
-                    rx[u] = v;
-                }
-            } else if (w_thread) {
-                if constexpr (Q8PAIR) {
-                    load_q8_pair(wrow, k0, w_part, rw[0]);
-                } else {
-#pragma unroll
-                    for (int u = 0; u < WU; ++u) load_w<TY>(wrow, k0, w_part * WU + u, rw[u]);
-                }
-            }
-        };
-        auto stash_chunk = [&](int k0, int b) {
-            if (!x_prod) {
-                if (w_thread) {
-                    if constexpr (Q8PAIR) {
-                        stash_q8_pair(rw[0], w_row, w_part, w_live, q_s[b], so_s[b]);
-                    } else {
-#pragma unroll
-                        for (int u = 0; u < WU; ++u)
-                            stash_w<TY>(rw[u], k0, w_row, w_part * WU + u, w_live, q_s[b], so_s[b]);
-                    }
-                }
-                return;
-            }
-            // x (scaled by 2^kn) to f16 hi / lo rows, the token's ratio and
-            // inverse scale, and (Q4_K) the group sums
-            auto emit = [&](int u, const f32x4& xv, float ratio, int kn, bool store_scale) {
-                const int i = ptid + XT * u, tok = i >> 5, k4 = i & 31;
-                if (store_scale && k4 == 0) {
-                    rs_s[b][tok] = ratio;
-                    iv_s[b][tok] = __builtin_amdgcn_ldexpf(1.f, -kn);
-                }
-                f16x4 hi, lo;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    hi[j] = (f16)xv[j];
-                    lo[j] = (f16)(xv[j] - (float)hi[j]);
-                }
-                const int off = sw(tok, k4 >> 1) + 4 * (k4 & 1);
-                *reinterpret_cast<f16x4*>(&xh_s[b][off]) = hi;
-                *reinterpret_cast<f16x4*>(&xl_s[b][off]) = lo;
-                if constexpr (OFFSET) {
-                    // the group's (scaled) x sum: eight consecutive lanes hold its 32 floats
-                    float sx = (xv[0] + xv[1]) + (xv[2] + xv[3]);
-                    sx = sum8(sx);
-                    if ((k4 & 7) == 0) xs_s[b][(k4 >> 3) * kGM + tok] = sx;
-                }
-            };
-            // Scale rule per (token, chunk), m the token's largest |x| in the
-            // chunk: k_c = 0 for m in [2^-6, 2^14), else 15 - e(m) with
-            // m < 2^e (so m 2^k_c lies in [2^14, 2^15)); no bound for m = 0
-            // or m not finite; k_t = min(k_t, k_c) from k_t = 100.  Once
-            // k_t = 0 and no |x| of the chunk reaches 2^14, k_t stays 0, so a
-            // wave whose tokens are all there skips the reduction and the
-            // scaling (the common case after the first chunk).
-            float ml[XU];
-            bool slow = false;
-#pragma unroll
-            for (int u = 0; u < XU; ++u) {
-                ml[u] = fmaxf(fmaxf(fabsf(rx[u][0]), fabsf(rx[u][1])), fmaxf(fabsf(rx[u][2]), fabsf(rx[u][3])));
-                slow |= !(ml[u] < 16384.f) || kx[u] != 0;
-            }
-            if (__builtin_amdgcn_ballot_w64(slow) == 0) {
-                // the wave's tokens keep scale 1: their (ratio, 1 / scale)
-                // entries need writing only if buffer b does not hold (1, 1)
-                const bool store = !ones[b];
-#pragma unroll
-                for (int u = 0; u < XU; ++u) emit(u, rx[u], 1.f, 0, store);
-                ones[b] = true;
-                return;
-            }
-            ones[b] = false;
-#pragma unroll
-            for (int u = 0; u < XU; ++u) {
-                // the token's 128 floats are on 32 consecutive lanes
-                const float m = max32(ml[u]);
-                int kn = kx[u];
-                if (m > 0.f && m <= 3.402823466e38f && !(m >= 0.015625f && m < 16384.f))
-                    kn = min(kn, 15 - __builtin_amdgcn_frexp_expf(m));
-                else if (m >= 0.015625f && m < 16384.f)
-                    kn = min(kn, 0);
-                const float ratio = __builtin_amdgcn_ldexpf(1.f, kn - kx[u]);
-                kx[u] = kn;
-                f32x4 xv;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) xv[j] = __builtin_amdgcn_ldexpf(rx[u][j], kn);
-                emit(u, xv, ratio, kn, true);
-            }
-        };
-        load_chunk(0);
-        stash_chunk(0, 0);
-        if (n_chunks > 1) load_chunk(kGK);  // in flight during chunk 0's MFMAs
-        __syncthreads();
-        for (int ch = 0; ch < n_chunks; ++ch) {
-            // Buffer (ch + 1) & 1 was last read in iteration ch - 1, before
-            // that iteration's barrier.
-            if (ch + 1 < n_chunks) {
-                stash_chunk((ch + 1) * kGK, (ch + 1) & 1);
-                if (ch + 2 < n_chunks) load_chunk((ch + 2) * kGK);
-            }
-            __syncthreads();
-        }
-        return;
-    }
-
-    const int lane = tid & 63, wave = tid >> 6;
-    const int wm = wave & 1, wn = wave >> 1;
+    const int t0 = tb * TM, r0 = rb * TN;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, hh = lane >> 5;
-    f32x16 y[kNTW];
-#pragma unroll
-    for (int n = 0; n < kNTW; ++n)
-#pragma unroll
-        for (int j = 0; j < 16; ++j) y[n][j] = 0.f;
+    const int kq = wave % KQ, wr = wave / KQ;
+    const int n_chunks = (a.in_dim + kGK - 1) / kGK;
 
-    __syncthreads();  // chunk 0 is stashed
-    // tokens of register j: 8 (j / 4) + 4 hh + j % 4 of the wave's 32
-    auto token_vals = [&](const float* src, f32x4 (&v)[4]) {
+    // ---- weights: piece p of the tile is piece p % PC of row p / PC.  Rows
+    // past the matrix repeat its last one; a piece that would reach past the
+    // matrix is put together from its 2-byte words.
+    auto fetch_w = [&](int ch) __attribute__((always_inline)) {
 #pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4) v[q4] = *reinterpret_cast<const f32x4*>(src + 32 * wm + 8 * q4 + 4 * hh);
+        for (int i = 0; i < (TN * PC + 511) / 512; ++i) {
+            const int n = wave + 8 * i, p = n * 64 + lane;
+            const int row = p / PC, c = p % PC;
+            if (row < TN && c < NPC) {
+                const size_t at = (size_t)min(r0 + row, a.rows - 1) * a.row_bytes + (size_t)ch * GTraits<TY>::bytes;
+                const size_t off = (at & ~(size_t)15) + 16 * c;
+                if (TY == kGQ4K || off + 16 <= a.w_bytes) {  // (a Q4_K row is whole pieces)
+                    dma16_lane(a.w + off, lds_addr(w_s) + n * 1024);
+                } else {
+#pragma unroll 1
+                    for (int u = 0; u < 8; ++u)
+                        *reinterpret_cast<uint16_t*>(w_s + p * 16 + 2 * u) =
+                            off + 2 * u + 2 <= a.w_bytes ? *reinterpret_cast<const uint16_t*>(a.w + off + 2 * u) : 0;
+                }
+            }
+        }
     };
+    // ---- x: token wave * NX + u, floats 4 lane .. + 3 of the chunk
+    f32x4 rx[NX];
+    int kx[NX];  // running scale exponents (100: no nonzero x yet)
+#pragma unroll
+    for (int u = 0; u < NX; ++u) kx[u] = 100;
+    auto load_x = [&](int ch) __attribute__((always_inline)) {
+        const int k = ch * kGK + 4 * lane;
+#pragma unroll
+        for (int u = 0; u < NX; ++u) {
+            // tokens past the batch repeat its last one and are not stored
+            const int tok = min(t0 + wave * NX + u, a.n_tok - 1);
+            rx[u] = *reinterpret_cast<const f32x4*>(a.x + (size_t)tok * a.in_dim + min(k, a.in_dim - 4));
+        }
+    };
+    int ones = 0;        // bit b: buffer b's ratios of this wave's tokens are 1 (uniform)
+    bool plain = false;  // every k_t of this wave's tokens is 0 (uniform)
+    // One token's floats to hi / lo rows, and (Q4_K) its group sums.
+    auto emit = [&](int b, int u, const f32x4& v) __attribute__((always_inline)) {
+        const int tok = wave * NX + u;
+        // hi once (pinned: the residual is taken against these very
+        // registers); in the order 0 2 1 3
+        f16x2 h0 = {(f16)v[0], (f16)v[2]}, h1 = {(f16)v[1], (f16)v[3]};
+        asm("" : "+v"(h0), "+v"(h1));
+        const f16x4 hi = {h0[0], h0[1], h1[0], h1[1]};
+        const f16x4 lo = {(f16)(v[0] - (float)h0[0]), (f16)(v[2] - (float)h0[1]), (f16)(v[1] - (float)h1[0]),
+                          (f16)(v[3] - (float)h1[1])};
+        const int at = tok * kGK + (((lane >> 1) ^ (tok & 15)) << 3) + 4 * (lane & 1);
+        *reinterpret_cast<f16x4*>(xh(b) + at) = hi;
+        *reinterpret_cast<f16x4*>(xl(b) + at) = lo;
+        if constexpr (OFFSET) {
+            // the sum of each group of 32: eight lanes hold its floats; lane 8 g
+            // stores the hi part, lane 8 g + 1 the lo part
+            const float sx = sum8((v[0] + v[1]) + (v[2] + v[3])) * 0.0625f;
+            const f16 h = (f16)sx;
+            const f16 l = (f16)(sx - (float)h);
+            if ((lane & 7) < 2) xs_s[b][tok * 16 + 8 * (lane & 1) + (lane >> 3)] = lane & 1 ? l : h;
+        }
+    };
+    auto stash_x = [&](int b, int ch) __attribute__((always_inline)) {
+        if ((TY == kGQ8_0 || g_dense<TY>()) && ch * kGK + 4 * lane >= a.in_dim) {  // K may end inside a chunk
+#pragma unroll
+            for (int u = 0; u < NX; ++u) rx[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        // once every k_t is 0 and no |x| reaches 2^14, nothing changes (a NaN
+        // passes through as it is)
+        float top = 0.f;
+#pragma unroll
+        for (int u = 0; u < NX; ++u) top = absmax3(rx[u][2], rx[u][3], absmax3(rx[u][0], rx[u][1], top));
+        if (plain && __builtin_amdgcn_ballot_w64(top >= 16384.f) == 0) {
+            if (!(ones >> b & 1)) {
+                if (lane < NX) rs_s[b][wave * NX + lane] = 1.f;
+                if (lane == 0) chg_s[b][wave] = 0;
+                ones |= 1 << b;
+            }
+        } else {
+            int changed = 0;
+            plain = true;
+#pragma unroll
+            for (int u = 0; u < NX; ++u) {
+                const float m = wave_max64(absmax3(rx[u][2], rx[u][3], absmax3(rx[u][0], rx[u][1], 0.f)));
+                int kn = kx[u];
+                if (m > 0.f && m <= 3.402823466e38f)
+                    kn = min(kn, m >= 0.015625f && m < 16384.f ? 0 : 14 - __builtin_amdgcn_frexp_expf(m));
+                const float ratio = kx[u] == 100 ? 1.f : __builtin_amdgcn_ldexpf(1.f, kn - kx[u]);
+                kx[u] = kn;
+                changed |= ratio != 1.f;
+                plain = plain && kn == 0;
+                if (lane == 0) rs_s[b][wave * NX + u] = ratio;
+            }
+            if (lane == 0) chg_s[b][wave] = changed;
+            ones &= ~(1 << b);
+        }
+#pragma unroll
+        for (int u = 0; u < NX; ++u) {
+            f32x4 v;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = __builtin_amdgcn_ldexpf(rx[u][j], kx[u]);
+            emit(b, u, v);
+        }
+    };
+
+    f32x16 y[TT][RT];
+#pragma unroll
+    for (int i = 0; i < TT; ++i)
+#pragma unroll
+        for (int n = 0; n < RT; ++n)
+#pragma unroll
+            for (int j = 0; j < 16; ++j) y[i][n][j] = 0.f;
+
+    fetch_w(0);
+    load_x(0);
+    stash_x(0, 0);
+    if (n_chunks > 1) load_x(1);
     for (int ch = 0; ch < n_chunks; ++ch) {
         const int b = ch & 1;
-        // y so far moves to each token's scale of this chunk (a power of two,
-        // exact; 1 unless the chunk lowered it).  Unconditional: a branch on
-        // a change flag costs the Q6_K consumer spills.
-        {
-            f32x4 rt[4];
-            token_vals(rs_s[b], rt);
+        // the chunk's bytes; this wave's x loads, issued after them, may still
+        // be in flight
+        if (ch > 0 && ch + 1 < n_chunks) wait_dma<NX>();
+        else wait_dma<0>();
+        __syncthreads();  // chunk ch is in LDS
+        WFrag<TY, KQ> w[RT];
 #pragma unroll
-            for (int n = 0; n < kNTW; ++n)
-#pragma unroll
-                for (int j = 0; j < 16; ++j) y[n][j] *= rt[j >> 2][j & 3];
+        for (int n = 0; n < RT; ++n) {
+            const int row = (wr * RT + n) * 32 + l32;
+            uint32_t sh = 0;
+            if constexpr (TY != kGQ4K && !g_dense<TY>())
+                sh = (uint32_t)((size_t)min(r0 + row, a.rows - 1) * a.row_bytes + (size_t)ch * GTraits<TY>::bytes) & 15;
+            if constexpr (g_dense<TY>()) w[n].load(w_s + row * STR, kq, hh, a.in_dim - ch * kGK);
+            else w[n].load(w_s + row * STR + sh, kq, hh);
         }
+        const int4 c0 = *reinterpret_cast<const int4*>(&chg_s[b][0]), c1 = *reinterpret_cast<const int4*>(&chg_s[b][4]);
+        const int chg = c0.x | c0.y | c0.z | c0.w | c1.x | c1.y | c1.z | c1.w;
+        __syncthreads();  // the weight bytes are in registers
+        if (ch + 1 < n_chunks) {
+            stash_x(b ^ 1, ch + 1);  // (before the transfers: its wait for x would wait for them too)
+            fetch_w(ch + 1);
+            if (ch + 2 < n_chunks) load_x(ch + 2);
+        }
+        // token of register j: 8 (j / 4) + 4 hh + j % 4 of the tile's 32
+        if (__builtin_amdgcn_readfirstlane(chg)) {
 #pragma unroll
-        for (int g = 0; g < NG; ++g) {
-            f32x16 acc[kNTW];
+            for (int i = 0; i < TT; ++i)
 #pragma unroll
-            for (int n = 0; n < kNTW; ++n)
+                for (int g = 0; g < 4; ++g) {
+                    const f32x4 r = *reinterpret_cast<const f32x4*>(&rs_s[b][32 * i + 8 * g + 4 * hh]);
 #pragma unroll
-                for (int j = 0; j < 16; ++j) acc[n][j] = 0.f;
+                    for (int n = 0; n < RT; ++n)
 #pragma unroll
-            for (int kk = 0; kk < KPG; ++kk) {
-                const int c = 2 * (g * KPG + kk) + hh;
-                const int xr = 32 * wm + l32;
-                const f16x8 ah = *reinterpret_cast<const f16x8*>(&xh_s[b][sw(xr, c)]);
-                const f16x8 al = *reinterpret_cast<const f16x8*>(&xl_s[b][sw(xr, c)]);
+                        for (int j = 0; j < 4; ++j) y[i][n][4 * g + j] *= r[j];
+                }
+        }
+        auto x_at = [&](const f16* xb, int i, int k) {
+            return *reinterpret_cast<const f16x8*>(xb + (32 * i + l32) * kGK + (((k >> 3) ^ (l32 & 15)) << 3));
+        };
+        f32x16 acc[TT][RT];
 #pragma unroll
-                for (int n = 0; n < kNTW; ++n) {
-                    const f16x8 bq = *reinterpret_cast<const f16x8*>(&q_s[b][sw(32 * kNTW * wn + 32 * n + l32, c)]);
-                    acc[n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bq, acc[n], 0, 0, 0);
-                    acc[n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, bq, acc[n], 0, 0, 0);
+        for (int s = 0; s < NK; ++s) {
+            const int k = WFrag<TY, KQ>::k_of(s, kq, hh);
+            f16x8 ah[TT], al[TT];
+#pragma unroll
+            for (int i = 0; i < TT; ++i) {
+                ah[i] = x_at(xh(b), i, k);
+                al[i] = x_at(xl(b), i, k);
+            }
+            const bool first = TY == kGQ8_0 ? s % 2 == 0 : s == 0;
+            if (first) {
+#pragma unroll
+                for (int i = 0; i < TT; ++i)
+#pragma unroll
+                    for (int n = 0; n < RT; ++n)
+#pragma unroll
+                        for (int j = 0; j < 16; ++j) acc[i][n][j] = 0.f;
+            }
+#pragma unroll
+            for (int n = 0; n < RT; ++n) {
+                f16x8 q, ql;
+                if constexpr (TY == kGQ6K) w[n].step(s, kq, q, ql);
+                else if constexpr (TY == kGQ4K) q = w[n].step(s, kq);
+                else q = w[n].step(s);
+#pragma unroll
+                for (int i = 0; i < TT; ++i) {
+                    acc[i][n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], q, acc[i][n], 0, 0, 0);
+                    acc[i][n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[i], q, acc[i][n], 0, 0, 0);
+                    if constexpr (TY == kGQ6K)
+                        acc[i][n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], ql, acc[i][n], 0, 0, 0);
                 }
             }
-            // tokens of register j: 8 (j / 4) + 4 hh + j % 4 of the wave's 32
-            f32x4 xs[4];
-            if constexpr (OFFSET) {
+            if constexpr (TY == kGQ8_0) {
+                if (s % 2 == 1) {  // a block is done
+                    // blocks past the matrix (K a half chunk short) hold other bytes
+                    const bool in = ch * kGK + (k & ~31) < a.in_dim;
 #pragma unroll
-                for (int q4 = 0; q4 < 4; ++q4)
-                    xs[q4] = *reinterpret_cast<const f32x4*>(&xs_s[b][g * kGM + 32 * wm + 8 * q4 + 4 * hh]);
-            }
+                    for (int n = 0; n < RT; ++n) {
+                        const float d = in ? w[n].d(s / 2) : 0.f;
 #pragma unroll
-            for (int n = 0; n < kNTW; ++n) {
-                const f32x2 so = so_s[b][(32 * kNTW * wn + 32 * n + l32) * NG + g];
+                        for (int i = 0; i < TT; ++i)
 #pragma unroll
-                for (int j = 0; j < 16; ++j) {
-                    float v = fmaf(so[0], acc[n][j], y[n][j]);
-                    if constexpr (OFFSET) v = fmaf(so[1], xs[j >> 2][j & 3], v);
-                    y[n][j] = v;
+                            for (int j = 0; j < 16; ++j) y[i][n][j] = fmaf(d, acc[i][n][j], y[i][n][j]);
+                    }
                 }
             }
         }
-        __syncthreads();  // chunk ch's operands are read; chunk ch + 1 is stashed
+        if constexpr (TY != kGQ8_0) {
+#pragma unroll
+            for (int n = 0; n < RT; ++n) {
+                const float d = w[n].d();
+#pragma unroll
+                for (int i = 0; i < TT; ++i)
+#pragma unroll
+                    for (int j = 0; j < 16; ++j) y[i][n][j] = fmaf(d, acc[i][n][j], y[i][n][j]);
+            }
+        }
+        if constexpr (OFFSET) {
+            if (kq == ch % KQ) {  // the ranges take the chunks' offsets in turn
+#pragma unroll
+                for (int n = 0; n < RT; ++n) {
+                    const f16x8 m = w[n].mins();
+                    const float dm = -16.f * w[n].dmin();
+#pragma unroll
+                    for (int i = 0; i < TT; ++i) {
+                        const f16x8 xs = *reinterpret_cast<const f16x8*>(&xs_s[b][(32 * i + l32) * 16 + 8 * hh]);
+                        f32x16 z;
+#pragma unroll
+                        for (int j = 0; j < 16; ++j) z[j] = 0.f;
+                        z = __builtin_amdgcn_mfma_f32_32x32x16_f16(xs, m, z, 0, 0, 0);
+#pragma unroll
+                        for (int j = 0; j < 16; ++j) y[i][n][j] = fmaf(dm, z[j], y[i][n][j]);
+                    }
+                }
+            }
+        }
     }
 
-    // back from each token's final x scale (the last chunk's buffer is not
-    // written again)
-    f32x4 iv[4];
-    token_vals(iv_s[(n_chunks - 1) & 1], iv);
+    // ---- the KQ partial sums, [range][token][row], through the x buffers;
+    // each staging wave knows its tokens' final scales
+    __syncthreads();
+    float* y_s = reinterpret_cast<float*>(xy_s);
 #pragma unroll
-    for (int n = 0; n < kNTW; ++n) {
-        const int r = r0 + 32 * kNTW * wn + 32 * n + l32;
-        if (r >= a.rows) continue;
+    for (int i = 0; i < TT; ++i)
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const int t = t0 + 32 * wm + 8 * (j >> 2) + 4 * hh + (j & 3);
-            if (t < a.n_tok) a.y[(size_t)t * a.rows + r] = y[n][j] * iv[j >> 2][j & 3];
-        }
+        for (int n = 0; n < RT; ++n)
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                const int tok = 32 * i + 8 * (j >> 2) + 4 * hh + (j & 3);
+                y_s[(kq * TM + tok) * TN + (wr * RT + n) * 32 + l32] = y[i][n][j];
+            }
+    if (lane == 0)
+#pragma unroll
+        for (int u = 0; u < NX; ++u) rs_s[0][wave * NX + u] = kx[u] == 100 ? 1.f : __builtin_amdgcn_ldexpf(1.f, -kx[u]);
+    __syncthreads();
+#pragma unroll
+    for (int i = tid; i < TM * TN; i += 512) {
+        const int tok = i / TN, row = i % TN;
+        if (t0 + tok >= a.n_tok || r0 + row >= a.rows) continue;
+        float v = y_s[i];
+#pragma unroll
+        for (int q = 1; q < KQ; ++q) v += y_s[q * TM * TN + i];
+        a.y[(size_t)(t0 + tok) * a.rows + r0 + row] = v * rs_s[0][tok];
     }
 }
 
+template <int TY, int TT, int RT, int WR>
+static void launch(const GemmArgs& a, hipStream_t st) {
+    constexpr int TM = 32 * TT, TN = 32 * RT * WR;
+    const long grid = ((long)a.n_tok + TM - 1) / TM * ((a.rows + TN - 1) / TN);
+    hipLaunchKernelGGL((qgemm_kernel<TY, TT, RT, WR>), dim3((unsigned)grid), dim3(512), 0, st, a);
+}
+
+// Tiles: 64 tokens (32 for a batch of at most 32), and 64 rows where they
+// still make a workgroup for every CU, else 32 (fewer rows raise the share of
+// x's staging, which every workgroup of a token block repeats; dense rows take
+// 32 beside 64 tokens, whose x leaves LDS for no more).
+constexpr long kCus = 256;
+static bool fills(const GemmArgs& a, int tm, int tn) {
+    return ((long)a.n_tok + tm - 1) / tm * ((a.rows + tn - 1) / tn) >= kCus;
+}
+template <int TY>
+static void launch_type(const GemmArgs& a, hipStream_t st) {
+    if (a.n_tok <= 32) {
+        if (fills(a, 32, 64)) launch<TY, 1, 1, 2>(a, st);
+        else launch<TY, 1, 1, 1>(a, st);
+    } else if (!g_dense<TY>() && fills(a, 64, 64)) {
+        if constexpr (!g_dense<TY>()) launch<TY, 2, 1, 2>(a, st);
+    } else {
+        launch<TY, 2, 1, 1>(a, st);
+    }
+}
+
+// qgemm_big.hip
+lmx_status qgemm_big(const lmx_qmv_desc* d, const void* w, const float* x, float* y, hipStream_t st);
+
 // y [n_tok, rows] = W x: one launch, W read once from HBM (each of the
-// ceil(n_tok / 64) token blocks of a row block reads it from L2 or the
-// last-level cache after the first).
+// token blocks of a row block reads it from L2 or the last-level cache after
+// the first).
 lmx_status qgemm(const lmx_qmv_desc* d, const void* w, const float* x, float* y, hipStream_t st) {
     size_t bb = 0, be = 0;
     switch (d->type) {
         case kGQ4K: bb = 144; be = 256; break;
         case kGQ6K: bb = 210; be = 256; break;
         case kGQ8_0: bb = 34; be = 32; break;
+        case kGF16: case kGBF16: bb = 2; be = 1; break;
         default: return LMX_E_UNSUPPORTED;
     }
-    if (d->in_dim % kGK || d->in_dim % be) return LMX_E_SHAPE;
+    if (d->in_dim % (be == 1 ? 64 : 128) || d->in_dim % be) return LMX_E_SHAPE;
     GemmArgs a{};
     a.w = static_cast<const uint8_t*>(w);
     a.x = x;
@@ -552,14 +661,17 @@ lmx_status qgemm(const lmx_qmv_desc* d, const void* w, const float* x, float* y,
     a.in_dim = (int)d->in_dim;
     a.n_tok = (int)d->n_tok;
     a.row_bytes = (size_t)d->in_dim / be * bb;
-    const long n_tb = ((long)d->n_tok + kGM - 1) / kGM, n_rb = ((long)d->rows + kGN - 1) / kGN;
-    if (n_tb * n_rb > INT32_MAX) return LMX_E_SHAPE;
-    const dim3 grid((unsigned)(n_tb * n_rb));
+    a.w_bytes = a.row_bytes * d->rows;
+    if (((long)d->n_tok + 31) / 32 * (((long)d->rows + 31) / 32) > INT32_MAX) return LMX_E_SHAPE;
+    // 64 x 128 tiles where they fill the GPU (see qgemm_big.hip)
+    if (be > 1 && d->n_tok > 32 && fills(a, 64, 128)) return qgemm_big(d, w, x, y, st);
     (void)hipGetLastError();
     switch (d->type) {
-        case kGQ4K: hipLaunchKernelGGL(qgemm_kernel<kGQ4K>, grid, dim3(g_threads<kGQ4K>()), 0, st, a); break;
-        case kGQ6K: hipLaunchKernelGGL(qgemm_kernel<kGQ6K>, grid, dim3(g_threads<kGQ6K>()), 0, st, a); break;
-        default: hipLaunchKernelGGL(qgemm_kernel<kGQ8_0>, grid, dim3(g_threads<kGQ8_0>()), 0, st, a); break;
+        case kGF16: launch_type<kGF16>(a, st); break;
+        case kGBF16: launch_type<kGBF16>(a, st); break;
+        case kGQ4K: launch_type<kGQ4K>(a, st); break;
+        case kGQ6K: launch_type<kGQ6K>(a, st); break;
+        default: launch_type<kGQ8_0>(a, st); break;
     }
     LMX_CHECK_LAUNCH();
     return LMX_OK;

@@ -47,9 +47,11 @@ struct QTraits;
 template <> struct QTraits<kQ4K> { static constexpr int unit = 64, bbytes = 144, belems = 256; };
 template <> struct QTraits<kQ6K> { static constexpr int unit = 64, bbytes = 210, belems = 256; };
 template <> struct QTraits<kQ8_0> { static constexpr int unit = 64, bbytes = 34, belems = 32; };
-template <> struct QTraits<kF32> { static constexpr int unit = 64, bbytes = 4, belems = 1; };
-template <> struct QTraits<kF16> { static constexpr int unit = 64, bbytes = 2, belems = 1; };
-template <> struct QTraits<kBF16> { static constexpr int unit = 64, bbytes = 2, belems = 1; };
+// dense rows: 16 bytes a unit, so that a wave's load covers 1 KB of a row
+// (units of 64 weights put its lanes 128 bytes apart: bf16 4096 x 4096 23 us)
+template <> struct QTraits<kF32> { static constexpr int unit = 4, bbytes = 4, belems = 1; };
+template <> struct QTraits<kF16> { static constexpr int unit = 8, bbytes = 2, belems = 1; };
+template <> struct QTraits<kBF16> { static constexpr int unit = 8, bbytes = 2, belems = 1; };
 
 // Weight bytes are streamed: read once, never reused.  LDS: the bytes were
 // staged in a wave's LDS slice first (qmatvec_lds_kernel).
@@ -306,46 +308,39 @@ __device__ __forceinline__ void unit_dot(const uint8_t* const (&row)[RW], int uw
             }
         }
     } else {
-        // dense rows: 64 consecutive weights
-        const int u = uw;
-        const float* xc = xs + 64 * ux;
+        // dense rows: U consecutive weights, one 16-byte load a row, every
+        // row's issued before the first is used
+        constexpr int U = QTraits<TY>::unit;
+        typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+        const float* xc = xs + U * ux;
+        u32x4 v[RW];
 #pragma unroll
-        for (int r = 0; r < RW; ++r) {
-            float wv[64];
-            if constexpr (TY == kF32) {
-                const float* p = reinterpret_cast<const float*>(row[r]) + 64 * u;
+        for (int r = 0; r < RW; ++r)
+            v[r] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(row[r] + (size_t)16 * uw));
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const f32x4 v = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p + 4 * i));
+        for (int t = 0; t < T; ++t) {
+            float xv[U];
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) wv[4 * i + j] = v[j];
-                }
-            } else {
-                const uint16_t* p = reinterpret_cast<const uint16_t*>(row[r]) + 64 * u;
+            for (int i = 0; i < U; i += 4) {
+                const f32x4 a = *reinterpret_cast<const f32x4*>(xc + t * in_dim + i);
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-                    const u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p + 8 * i));
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        if constexpr (TY == kF16) {
-                            wv[8 * i + 2 * j] = f16_lo(v[j]);
-                            wv[8 * i + 2 * j + 1] = f16_hi(v[j]);
-                        } else {  // bf16: the top half of an f32
-                            wv[8 * i + 2 * j] = __builtin_bit_cast(float, v[j] << 16);
-                            wv[8 * i + 2 * j + 1] = __builtin_bit_cast(float, v[j] & 0xFFFF0000u);
-                        }
-                    }
-                }
+                for (int j = 0; j < 4; ++j) xv[i + j] = a[j];
             }
 #pragma unroll
-            for (int t = 0; t < T; ++t) {
+            for (int r = 0; r < RW; ++r) {
                 float s = 0.f;
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const f32x4 a = *reinterpret_cast<const f32x4*>(xc + t * in_dim + 4 * i);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) s = fmaf(wv[4 * i + j], a[j], s);
+                for (int j = 0; j < 4; ++j) {
+                    const uint32_t wv = v[r][j];
+                    if constexpr (TY == kF32) {
+                        s = fmaf(__builtin_bit_cast(float, wv), xv[j], s);
+                    } else if constexpr (TY == kF16) {
+                        s = fmaf(f16_lo(wv), xv[2 * j], s);
+                        s = fmaf(f16_hi(wv), xv[2 * j + 1], s);
+                    } else {  // bf16: the top half of an f32
+                        s = fmaf(__builtin_bit_cast(float, wv << 16), xv[2 * j], s);
+                        s = fmaf(__builtin_bit_cast(float, wv & 0xFFFF0000u), xv[2 * j + 1], s);
+                    }
                 }
                 acc[r][t] += s;
             }
@@ -396,6 +391,8 @@ __global__ __launch_bounds__(kQmvWaves * 64) void qmatvec_kernel(QmvArgs a) {
         for (int r = 0; r < kQmvRows; ++r)
 #pragma unroll
             for (int t = 0; t < T; ++t) acc[r][t] = 0.f;
+        constexpr int UNROLL = QTraits<TY>::unit < 64 ? 4 : 1;  // dense units are one load a row
+#pragma unroll UNROLL
         for (int u = lane; u < n_units; u += 64) unit_dot<TY, T, false, kQmvRows>(row, u, u, xs, a.in_dim, acc);
 #pragma unroll
         for (int r = 0; r < kQmvRows; ++r) {
@@ -543,17 +540,30 @@ static lmx_status launch_type(const QmvArgs& a, int T, hipStream_t st) {
 // qgemm.hip: the matrix-core GEMM for batches of tokens
 lmx_status qgemm(const lmx_qmv_desc* d, const void* w, const float* x, float* y, hipStream_t st);
 
-// From this many tokens the GEMM takes the k-quant formats (the reference's
-// GEMM_MIN_TOKENS, crates/gpu/src/lib.rs:1083): one launch reads W once.
-constexpr uint32_t kGemmMinTokens = 16;
+// Tokens from which the GEMM is the faster one.  It reads W once and takes about
+// the same time up to 32 tokens, the matvec a launch per four.  At in_dim 4096,
+// us at 4 / 8 / 12 tokens against the GEMM: Q6_K 1024 rows 8 / 16 / 24 : 28,
+// 4096 rows 17 / 33 / 49 : 29; Q8_0 4096 rows 26 / 50 / 74 : 23; bf16 4096
+// rows 13 / 26 / 38 : 26.  So: with the third launch, with the second where rows or
+// bytes are many, with the fourth for a short Q6_K matrix.  Q4_K waits for the
+// reference's 16: the GEMM's offset term, split into f16 parts, is 2.0e-7 from
+// the exact sums where the matvec is 1.6e-7 (the other types' GEMM is the
+// closer one).  fp32 weights stay with the matvec.
+static uint32_t gemm_min_tokens(uint32_t type, uint32_t rows) {
+    if (type == kF32) return UINT32_MAX;
+    if (type == kQ4K) return 16;
+    if (type == kF16 || type == kBF16) return 9;
+    if (type == kQ6K && rows < 2048) return 13;
+    return rows >= (type == kQ8_0 ? 2048u : 8192u) ? 5 : 9;
+}
 
 // Host side: tokens go in tiles of up to kQmvMaxTok (each tile re-reads W),
 // or to the GEMM.
 lmx_status qmatvec(const lmx_qmv_desc* d, const void* w, const float* x, float* y, hipStream_t st) {
-    if (d->n_tok >= kGemmMinTokens && d->in_dim % 128 == 0 &&
-        (d->type == kQ4K || d->type == kQ6K || d->type == kQ8_0))
+    const bool dense = d->type == kF32 || d->type == kF16 || d->type == kBF16;
+    if (d->n_tok >= gemm_min_tokens(d->type, d->rows) && (dense || d->in_dim % 128 == 0))
         return qgemm(d, w, x, y, st);
-    int unit = 0;
+    int unit = 0;  // of the shape check
     size_t bb = 0, be = 0;
     switch (d->type) {
         case kQ4K: unit = 64; bb = 144; be = 256; break;

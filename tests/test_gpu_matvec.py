@@ -163,3 +163,41 @@ def test_gemm_x_range(name):
         err = np.abs(got[t] - ref[t]).max()
         scale = np.abs(ref[t]).max()
         assert err <= 3e-5 * scale, f"{name} token {t} (kind {t % 5}): max err {err} vs max |ref| {scale}"
+
+
+@pytest.mark.parametrize("name,in_dim", [("bf16", 320), ("bf16", 2560), ("f16", 192), ("f16", 1024)])
+@pytest.mark.parametrize("rows,n_tok", [(37, 16), (70, 33), (200, 65), (1, 130)])
+def test_gemm_dense_edges(name, in_dim, rows, n_tok):
+    # dense rows through the GEMM: K ending inside a 256-weight chunk, rows and
+    # tokens off the 32- and 64-wide tiles
+    run(name, rows, in_dim, n_tok, seed=90 + rows + n_tok)
+
+
+@pytest.mark.parametrize("name,in_dim", [("q4_k", 768), ("q6_k", 256), ("q6_k", 1280), ("q8_0", 384)])
+@pytest.mark.parametrize("rows,n_tok", [(1, 16), (33, 32), (65, 64), (8200, 40), (16500, 17)])
+def test_gemm_row_tiles(name, in_dim, rows, n_tok):
+    # each tile of the dispatch: 32 and 64 rows beside 32 and 64 tokens, 64 x 128
+    # for the largest grids; the last row's bytes end the matrix
+    run(name, rows, in_dim, n_tok, seed=120 + rows % 97 + n_tok)
+
+
+def test_gemm_bf16_weight_range():
+    # a chunk of a row is scaled by its own largest weight: rows and chunks of
+    # very different sizes, zeros, and a row that falls by 2^-20 along a chunk
+    rows, in_dim, n_tok = 40, 512, 20
+    rng = np.random.default_rng(7)
+    w = rng.standard_normal((rows, in_dim)).astype(np.float32)
+    w[1] *= 1e-30
+    w[2] *= 1e30
+    w[3, 256:] *= 1e-12
+    w[4] = 0.0
+    w[5] *= np.exp2(-20.0 * np.arange(in_dim) / 256).astype(np.float32)
+    bits = (w.view(np.uint32) >> 16).astype(np.uint16)
+    w64 = (bits.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+    x = oracle.normal(91, (n_tok, in_dim))
+    y = lmx.matvec(torch.from_numpy(bits.view(np.uint8).reshape(-1).copy()).cuda(), torch.from_numpy(x).cuda(),
+                   qtype="bf16", rows=rows, in_dim=in_dim)
+    torch.cuda.synchronize()
+    got, ref = y.cpu().numpy().astype(np.float64), x.astype(np.float64) @ w64.T
+    for r in range(rows):  # each row against its own scale
+        assert np.abs(got[:, r] - ref[:, r]).max() <= 3e-6 * np.abs(ref[:, r]).max(), r
