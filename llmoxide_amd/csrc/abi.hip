@@ -25,6 +25,7 @@ lmx_status decode_batched(const lmx_attn_params* p, int n_seq, int max_ctx, cons
                           lmx_dtype q_dt, float* out, void* ws, size_t ws_bytes, hipStream_t st);
 // attn_prefill.hip
 bool prefill_supported(const lmx_attn_params* p, lmx_dtype q_dt);
+size_t prefill_needed_bytes(const lmx_attn_params* p);
 size_t prefill_workspace_bytes(const lmx_attn_params* p);
 lmx_status prefill_fwd(const lmx_attn_params* p, const AttnIo& io, const void* q, lmx_dtype q_dt,
                        const void* k_cache, const void* v_cache, const void* k_cur, const void* v_cur,
@@ -67,6 +68,7 @@ static bool overlaps(const void* a, size_t na, const void* b, size_t nb) {
 
 // attn_pad.hip: head sizes outside the kernels' set, through padded copies
 bool native_head_dim(uint32_t hd);
+size_t padded_needed_bytes(const lmx_attn_params* p);
 size_t padded_workspace_bytes(const lmx_attn_params* p);
 lmx_status padded_attn(const lmx_attn_params* p, const AttnIo& io, const void* q, lmx_dtype q_dt,
                        const void* k_cache, const void* v_cache, const void* k_cur, const void* v_cur,
@@ -392,21 +394,34 @@ lmx_status lmx_attn_fwd_ext(const lmx_attn_params* p, const lmx_attn_ext* x, con
                        (hipStream_t)stream);
 }
 
+// The workspace without which lmx_attn_fwd refuses a call.
+static size_t needed_bytes(const lmx_attn_params* p) {
+    if (!native_head_dim(p->head_dim)) return padded_needed_bytes(p);
+    size_t need = 0;
+    for (lmx_dtype dt : {LMX_F32, LMX_F16}) {
+        const size_t b = use_split_k(p, dt) ? decode_workspace_bytes(p) : prefill_needed_bytes(p);
+        if (b > need) need = b;
+    }
+    return need;
+}
+
 lmx_status lmx_attn_fwd_noalloc(const lmx_attn_params* p, const void* q, lmx_dtype q_dt,
                                 const void* k_cache, const void* v_cache, lmx_dtype kv_dt,
                                 const void* k_cur, const void* v_cur, float* out,
                                 lmx_stream stream) {
     lmx_status s = check_attn_params(p);
     if (s != LMX_OK) return s;
-    const size_t need = lmx_attn_workspace_bytes(p);
+    const size_t need = needed_bytes(p);
     if (need > kScratchBytes) return LMX_E_WORKSPACE;
+    // A call that can use more than it must have gets the whole scratch.
+    const bool use = lmx_attn_workspace_bytes(p) > 0;
     void* ws = nullptr;
-    if (need > 0) {
+    if (use) {
         s = scratch_of_stream_device((hipStream_t)stream, &ws);
         if (s != LMX_OK) return s;
     }
     return lmx_attn_fwd_ext(p, nullptr, q, q_dt, k_cache, v_cache, kv_dt, k_cur, v_cur, out, ws,
-                            need > 0 ? kScratchBytes : 0, stream);
+                            use ? kScratchBytes : 0, stream);
 }
 
 size_t lmx_attn_decode_batched_workspace_bytes(const lmx_attn_params* p, int32_t n_seq,

@@ -20,6 +20,8 @@
 // Those dims are copied to the caller's out, where the output gate, if any,
 // is applied.  The copies are HBM-bound passes of their own (read + write of
 // each padded buffer); the attention kernels run as at the native size.
+#include <algorithm>
+
 #include "common.hpp"
 
 namespace lmx {
@@ -31,6 +33,7 @@ lmx_status prefill_fwd(const lmx_attn_params* p, const AttnIo& io, const void* q
                        const void* k_cache, const void* v_cache, const void* k_cur, const void* v_cur,
                        float* out, void* ws, size_t ws_bytes, hipStream_t st);
 size_t decode_workspace_bytes(const lmx_attn_params* p);
+size_t prefill_needed_bytes(const lmx_attn_params* p);
 size_t prefill_workspace_bytes(const lmx_attn_params* p);
 bool use_split_k(const lmx_attn_params* p, lmx_dtype q_dt);
 
@@ -57,16 +60,19 @@ static lmx_attn_params padded_params(const lmx_attn_params* p) {
 }
 
 struct PadLayout {
-    size_t inner, q, kv, cur, out, total;  // byte offsets of each buffer, and the total
+    // byte offsets of each buffer; more is a prefill's larger workspace, which
+    // takes inner's place in a call given all of total
+    size_t inner, q, kv, cur, out, more, total;
 };
 
 static PadLayout pad_layout(const lmx_attn_params* p) {
     const lmx_attn_params pp = padded_params(p);
     const size_t hp = pp.head_dim;
-    size_t inner = 0;
+    size_t inner = 0, more = 0;
     for (lmx_dtype dt : {LMX_F32, LMX_F16}) {
-        const size_t b = use_split_k(&pp, dt) ? decode_workspace_bytes(&pp) : prefill_workspace_bytes(&pp);
-        if (b > inner) inner = b;
+        const bool dec = use_split_k(&pp, dt);
+        inner = std::max(inner, dec ? decode_workspace_bytes(&pp) : prefill_needed_bytes(&pp));
+        if (!dec) more = std::max(more, prefill_workspace_bytes(&pp));
     }
     PadLayout L;
     L.inner = 0;
@@ -74,10 +80,12 @@ static PadLayout pad_layout(const lmx_attn_params* p) {
     L.kv = L.q + up256((size_t)p->n_tokens * p->n_heads * hp * 4);  // room for an fp32 query
     L.cur = L.kv + 2 * up256((size_t)pp.n_slots * pp.kv_dim * 2);
     L.out = L.cur + 2 * up256((size_t)p->n_tokens * pp.kv_dim * 2);
-    L.total = L.out + up256((size_t)p->n_tokens * p->n_heads * hp * 4);
+    L.more = L.out + up256((size_t)p->n_tokens * p->n_heads * hp * 4);
+    L.total = L.more + (more > inner ? up256(more) : 0);
     return L;
 }
 
+size_t padded_needed_bytes(const lmx_attn_params* p) { return pad_layout(p).more; }
 size_t padded_workspace_bytes(const lmx_attn_params* p) { return pad_layout(p).total; }
 
 // dst[r][h][0 .. hp) = src[r * row_stride + h * head_stride + 0 .. hd), zero
@@ -124,7 +132,7 @@ lmx_status padded_attn(const lmx_attn_params* p, const AttnIo& io, const void* q
                        const void* k_cache, const void* v_cache, const void* k_cur, const void* v_cur,
                        float* out, void* ws, size_t ws_bytes, hipStream_t st) {
     const PadLayout L = pad_layout(p);
-    if (!ws || ws_bytes < L.total) return LMX_E_WORKSPACE;
+    if (!ws || ws_bytes < L.more) return LMX_E_WORKSPACE;
     if (((uintptr_t)ws & 255) != 0) return LMX_E_ALIGN;
     const lmx_attn_params pp = padded_params(p);
     const int hd = (int)p->head_dim, hp = (int)pp.head_dim;
@@ -159,9 +167,11 @@ lmx_status padded_attn(const lmx_attn_params* p, const AttnIo& io, const void* q
     }
     if (hipGetLastError() != hipSuccess) return LMX_E_LAUNCH;
     const AttnIo pio{hp, hp, nullptr};
+    const bool all = L.total > L.more && ws_bytes >= L.total;
+    const size_t iw = all ? L.more : L.inner, iw_bytes = all ? L.total - L.more : L.q;
     const lmx_status s = use_split_k(&pp, q_dt)
                              ? decode_fwd(&pp, pio, qp, q_dt, kp, vp, kcp, vcp, op, w + L.inner, L.q, st)
-                             : prefill_fwd(&pp, pio, qp, q_dt, kp, vp, kcp, vcp, op, w + L.inner, L.q, st);
+                             : prefill_fwd(&pp, pio, qp, q_dt, kp, vp, kcp, vcp, op, w + iw, iw_bytes, st);
     if (s != LMX_OK) return s;
     hipLaunchKernelGGL(unpad_out_kernel, dim3(grid_for(t * H * hd / 4)), dim3(256), 0, st, op, out, t * H, hd, hp,
                        io.gate, io.gate_stride);

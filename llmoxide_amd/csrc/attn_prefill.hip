@@ -14,8 +14,8 @@
 //
 // Three kernels here share these tiles (head_dim 64 and 128; 256 and 512 are
 // attn_prefill_wide.hip's).  attn_prefill_kernel: workgroup = 4 waves x 32
-// query rows of one query head, two workgroups per CU.  The ping-pong
-// kernel (head_dim 128, long batches): 8 waves x 32 rows, one workgroup per
+// query rows of one query head, two workgroups per CU (fp32 queries at
+// head_dim 128: one).  The ping-pong kernel (head_dim 128, long batches): 8 waves x 32 rows, one workgroup per
 // CU, the two waves of each SIMD kept half a tile apart so one's MFMAs run
 // beside the other's softmax.  The key-halves kernel (short batches): 64
 // query rows, two wave pairs on the two halves of the key range, merged in
@@ -101,6 +101,60 @@ __device__ __forceinline__ void qk_tile(const f16* Ks, const f16x8 (&qf)[HD / 16
     }
 }
 
+// A query row as the B operands of its k-steps: qf[ks][j] is element
+// ks*16 + j after off (j < 8).  f16 queries are used as given and *c_sc stays
+// c = scale * log2(e).  An fp32 query has c 2^S folded in before its f16
+// rounding (the row's largest |x c 2^S| in [2^14, 2^15); 2^S = 1 for an
+// all-zero or non-finite row); its residual's fragments go to ql_row (LDS)
+// and *c_sc becomes 2^-S, which scales the scores back (qk_tile).
+template <typename QT, int HD>
+__device__ __forceinline__ void load_q(const void* q, size_t off, f16x8 (&qf)[HD / 16], f16* ql_row, float* c_sc) {
+    constexpr int KSTEPS = HD / 16;
+    if constexpr (sizeof(QT) == 2) {
+#pragma unroll
+        for (int ks = 0; ks < KSTEPS; ++ks)
+            qf[ks] = *reinterpret_cast<const f16x8*>(reinterpret_cast<const f16*>(q) + off + ks * 16);
+    } else {
+        const float* row = reinterpret_cast<const float*>(q) + off;
+        float m = 0.f;
+#pragma unroll
+        for (int ks = 0; ks < KSTEPS; ++ks) {
+            const f32x4 x0 = *reinterpret_cast<const f32x4*>(row + ks * 16);
+            const f32x4 x1 = *reinterpret_cast<const f32x4*>(row + ks * 16 + 4);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) m = fmaxf(m, fmaxf(fabsf(x0[j]), fabsf(x1[j])));
+        }
+        m = fmaxf(m, shfl_xor(m, 32)) * *c_sc;  // the row's two halves
+        const int S = (m > 0.f && m <= 3.402823466e38f) ? 15 - __builtin_amdgcn_frexp_expf(m) : 0;
+        const float qc = *c_sc * __builtin_amdgcn_ldexpf(1.f, S);  // x c 2^S
+        *c_sc = __builtin_amdgcn_ldexpf(1.f, -S);
+#pragma unroll
+        for (int ks = 0; ks < KSTEPS; ++ks) {
+            const f32x4 x0 = *reinterpret_cast<const f32x4*>(row + ks * 16);
+            const f32x4 x1 = *reinterpret_cast<const f32x4*>(row + ks * 16 + 4);
+            // y = x c 2^S once, and the residual taken against the very
+            // registers the MFMA reads: with contraction on, the compiler
+            // otherwise forms the residual's hi as one fused
+            // multiply-convert (one rounding) and the MFMA operand's as
+            // multiply then convert (two), which differ by an f16 ulp
+            // where the fp32 product is a tie.
+            float y[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                y[j] = (j < 4 ? x0[j] : x1[j - 4]) * qc;
+                asm volatile("" : "+v"(y[j]));
+                qf[ks][j] = (f16)y[j];
+            }
+            asm volatile("" : "+v"(qf[ks]));
+            f16x8 lo;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) lo[j] = (f16)(y[j] - (float)qf[ks][j]);
+            *reinterpret_cast<f16x8*>(ql_row + ks * 16) = lo;
+        }
+    }
+    settle_q(qf);
+}
+
 // A raw buffer resource over p (dword 3 = 0x00020000: 32-bit data format, the
 // form raw buffer loads take on gfx9 parts) with 2^31 - 1 bytes of range,
 // which the rows of one K/V tile never leave.  p must be wave-uniform: it is
@@ -151,10 +205,13 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PrefillArgs a) {
     // Query tiles heaviest first (causal work grows with qt).  When the whole
     // grid is resident at once (two workgroups per CU), the second half is
     // walked lightest first, so the two workgroups a CU receives pair a heavy
-    // tile with a light one instead of two of nearly the same weight.
+    // tile with a light one instead of two of nearly the same weight.  Not
+    // where the residuals leave a CU room for one workgroup: the CU that took
+    // a heavy tile would then get the second half's heaviest.
     const int pos = rem / (hgroups * n_split);
     const int half = (a.n_qtiles + 1) / 2;
-    const bool fold = nblk <= 2 * kPfCus;
+    constexpr bool kTwo = sizeof(K_s) + sizeof(Vt_s) + sizeof(QL_s) <= 80 * 1024;  // workgroups a CU holds
+    const bool fold = kTwo && nblk <= 2 * kPfCus;
     const int qt = (fold && pos >= half) ? pos - half : a.n_qtiles - 1 - pos;
     const int rem2 = rem % (hgroups * n_split);
     const int sp = rem2 % n_split;
@@ -180,78 +237,12 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PrefillArgs a) {
     const int my_lo = qvalid ? vis_lo(qpos, w) : 1;
     const int my_hi = qvalid ? vis_hi(qpos, w, a.bidi, end) : 0;
 
-    // Q as the B operand: lane holds Q[qrow][ks*16 + 8*hh + j], j < 8.  An fp32
-    // query has c = scale * log2(e) folded in before its f16 rounding, and its
-    // residual is the second operand (kQlo); an f16 query is used as given and
-    // qk_tile scales its scores.
+    // Q as the B operand: lane holds Q[qrow][ks*16 + 8*hh + j], j < 8.
     f16x8 qf[KSTEPS];
     const size_t qoff = ((size_t)(qvalid ? qrow : 0) * a.H + h) * a.q_stride + 8 * hh;
-    const float* qrow32 = reinterpret_cast<const float*>(a.q) + qoff;
     f16* ql_row = &QL_s[kQlo ? (wave * 32 + l32) * QLPAD + 8 * hh : 0];
-    // fp32 queries: c 2^S folded into Q (the row's largest |x c 2^S| in
-    // [2^14, 2^15); 2^S = 1 for an all-zero or non-finite row), and the
-    // scores scaled back by c_sc = 2^-S; f16 queries: Q as given, c_sc = c.
-    float qs = 1.f, c_sc = a.c;
-    if constexpr (kQlo) {
-        float m = 0.f;
-#pragma unroll
-        for (int ks = 0; ks < KSTEPS; ++ks) {
-            const f32x4 x0 = *reinterpret_cast<const f32x4*>(qrow32 + ks * 16);
-            const f32x4 x1 = *reinterpret_cast<const f32x4*>(qrow32 + ks * 16 + 4);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) m = fmaxf(m, fmaxf(fabsf(x0[j]), fabsf(x1[j])));
-        }
-        m = fmaxf(m, shfl_xor(m, 32)) * a.c;  // the row's two halves
-        const int S = (m > 0.f && m <= 3.402823466e38f) ? 15 - __builtin_amdgcn_frexp_expf(m) : 0;
-        qs = __builtin_amdgcn_ldexpf(1.f, S);
-        c_sc = __builtin_amdgcn_ldexpf(1.f, -S);
-    }
-    const float qc = a.c * qs;  // fp32 queries: x c 2^S
-    {
-#pragma unroll
-        for (int ks = 0; ks < KSTEPS; ++ks) {
-            float x[8];
-            if constexpr (sizeof(QT) == 2) {
-                const f16x8 q8 = *reinterpret_cast<const f16x8*>(reinterpret_cast<const f16*>(a.q) + qoff + ks * 16);
-#pragma unroll
-                for (int j = 0; j < 8; ++j) x[j] = (float)q8[j];
-            } else {
-                const f32x4 x0 = *reinterpret_cast<const f32x4*>(qrow32 + ks * 16);
-                const f32x4 x1 = *reinterpret_cast<const f32x4*>(qrow32 + ks * 16 + 4);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    x[j] = x0[j];
-                    x[4 + j] = x1[j];
-                }
-            }
-            if constexpr (kExact) {
-#pragma unroll
-                for (int j = 0; j < 8; ++j) qf[ks][j] = (f16)x[j];
-            } else {
-                // y = x c 2^S once, and the residual taken against the very
-                // registers the MFMA reads: with contraction on, the compiler
-                // otherwise forms the residual's hi as one fused
-                // multiply-convert (one rounding) and the MFMA operand's as
-                // multiply then convert (two), which differ by an f16 ulp
-                // where the fp32 product is a tie.
-                float y[8];
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    y[j] = x[j] * qc;
-                    asm volatile("" : "+v"(y[j]));
-                    qf[ks][j] = (f16)y[j];
-                }
-                asm volatile("" : "+v"(qf[ks]));
-                {
-                    f16x8 lo;
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) lo[j] = (f16)(y[j] - (float)qf[ks][j]);
-                    *reinterpret_cast<f16x8*>(ql_row + ks * 16) = lo;
-                }
-            }
-        }
-        settle_q(qf);
-    }
+    float c_sc = a.c;
+    load_q<QT, HD>(a.q, qoff, qf, ql_row, &c_sc);
     // The residual's fragment of k-step ks (read after the first barrier of
     // the key loop, which orders the stores above before it).
     auto ql = [&](int ks) -> f16x8 {
@@ -958,7 +949,7 @@ constexpr int kPpBM = 256;  // query rows per workgroup: 8 waves x 32
 
 template <typename QT, int HD, bool LIN>
 __global__ __launch_bounds__(512, 1) void attn_prefill_pp_kernel(PrefillArgs a) {
-    constexpr bool kExact = sizeof(QT) == 2;  // f16 queries: scale applied in fp32 (qk_tile)
+    constexpr bool kQlo = sizeof(QT) == 4;  // fp32 queries carry an f16 residual (qk_tile)
     constexpr int BN = 64;
     constexpr int KB = BN / 32;      // 32-key MFMA blocks per tile
     constexpr int PST = BN / 16;     // 16-key P.V k-steps per tile
@@ -969,15 +960,20 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_pp_kernel(PrefillArgs a) 
     static_assert(HD <= 128, "two waves per SIMD");
     __shared__ __attribute__((aligned(16))) f16 K_s[2 * BN * KPAD];
     __shared__ __attribute__((aligned(16))) f16 Vt_s[2 * HD * VPAD];
+    // fp32 queries' residuals, one padded row per query (as above)
+    constexpr int QLPAD = HD + 8;
+    __shared__ __attribute__((aligned(16))) f16 QL_s[kQlo ? kPpBM * QLPAD : 8];
 
     // The workgroup's gp query heads share kv head kvh, 256 / gp rows each.
     const int nblk = gridDim.x;
     const int logical = xcd_remap(blockIdx.x, nblk);
     const int gp = a.gp, hgroups = a.G / gp;
-    const int per_kvh = a.n_qtiles * hgroups;
+    const int n_split = a.n_split;
+    const int per_kvh = a.n_qtiles * hgroups * n_split;
     const int kvh = logical / per_kvh;
     const int rem = logical - kvh * per_kvh;
-    const int qt = a.n_qtiles - 1 - rem / hgroups;
+    const int qt = a.n_qtiles - 1 - rem / (hgroups * n_split);  // heaviest first
+    const int sp = rem % n_split;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -991,7 +987,7 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_pp_kernel(PrefillArgs a) 
     // The groups take alternate 32-row blocks, so the two waves of a SIMD
     // have nearly the same causal key range (and, with gp = 4, one head).
     const int blk = 2 * (wave & 3) + grp, bph = 8 / gp;  // 32-row blocks per head
-    const int h = kvh * a.G + (rem % hgroups) * gp + blk / bph;
+    const int h = kvh * a.G + (rem / n_split % hgroups) * gp + blk / bph;
     const int qw0 = q0 + 32 * (blk % bph);
 
     const int qrow = qw0 + l32;
@@ -1001,37 +997,26 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_pp_kernel(PrefillArgs a) 
     const int my_hi = qvalid ? vis_hi(qpos, w, a.bidi, end) : 0;
 
     f16x8 qf[KSTEPS];
-    {
-        const size_t qoff = ((size_t)(qvalid ? qrow : 0) * a.H + h) * a.q_stride + 8 * hh;
-#pragma unroll
-        for (int ks = 0; ks < KSTEPS; ++ks) {
-            float x[8];
-            if constexpr (sizeof(QT) == 2) {
-                const f16x8 q8 = *reinterpret_cast<const f16x8*>(reinterpret_cast<const f16*>(a.q) + qoff + ks * 16);
-#pragma unroll
-                for (int j = 0; j < 8; ++j) x[j] = (float)q8[j];
-            } else {
-                const float* qp = reinterpret_cast<const float*>(a.q) + qoff + ks * 16;
-                const f32x4 x0 = *reinterpret_cast<const f32x4*>(qp);
-                const f32x4 x1 = *reinterpret_cast<const f32x4*>(qp + 4);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    x[j] = x0[j];
-                    x[4 + j] = x1[j];
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < 8; ++j) qf[ks][j] = (f16)(kExact ? x[j] : x[j] * a.c);
-        }
-        settle_q(qf);
-    }
+    const size_t qoff = ((size_t)(qvalid ? qrow : 0) * a.H + h) * a.q_stride + 8 * hh;
+    f16* ql_row = &QL_s[kQlo ? (wave * 32 + l32) * QLPAD + 8 * hh : 0];
+    float c_sc = a.c;
+    load_q<QT, HD>(a.q, qoff, qf, ql_row, &c_sc);
+    // Each wave reads back only the residuals its own lanes stored.
+    auto ql = [&](int ks) -> f16x8 {
+        if constexpr (kQlo) return *reinterpret_cast<const f16x8*>(ql_row + ks * 16);
+        else return f16x8{};
+    };
 
     // ---- key tiles of the workgroup, and the wave's own run of them
     const int q_last = min(q0 + bm, t) - 1;
     const int wg_lo = vis_lo(base + q0, w);
     const int wg_hi = vis_hi(base + q_last, w, a.bidi, end);
-    const int kt_begin = (wg_lo / BN) * BN;
-    const int n_t = wg_lo <= wg_hi ? (wg_hi - kt_begin) / BN + 1 : 0;
+    const int kt_all = (wg_lo / BN) * BN;
+    const int n_t_all = wg_lo <= wg_hi ? (wg_hi - kt_all) / BN + 1 : 0;
+    // this split's share of the tiles (empty past the last one)
+    const int cs = (n_t_all + n_split - 1) / n_split;
+    const int kt_begin = kt_all + sp * cs * BN;
+    const int n_t = max(0, min(cs, n_t_all - sp * cs));
     const bool wave_live = qw0 < t;
     const int wq_last = min(qw0 + 31, t - 1);
     const int wv_lo_max = wave_live ? vis_lo(base + wq_last, w) : 0;           // largest lo
@@ -1041,8 +1026,8 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_pp_kernel(PrefillArgs a) 
         const int wv_lo = vis_lo(base + qw0, w);
         const int wv_hi = min(vis_hi(base + wq_last, w, a.bidi, end), wg_hi);
         if (wv_lo <= wv_hi) {
-            wi0 = (wv_lo - kt_begin) / BN;
-            wi1 = (wv_hi - kt_begin) / BN;
+            wi0 = max((wv_lo - kt_all) / BN - sp * cs, 0);
+            wi1 = min((wv_hi - kt_all) / BN - sp * cs, n_t - 1);
         }
     }
     const int cur_begin = (!LIN && a.k_cur) ? base : INT_MAX;
@@ -1166,7 +1151,7 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_pp_kernel(PrefillArgs a) 
     // S^T - mb = K Q^T - mb; mb is the running max once one is set.
     auto qk = [&](const f16* Ks) {
         mb = m_run > -1e29f ? m_run : 0.f;
-        qk_tile<HD, KB, KPAD, kExact>(Ks, qf, s, mb, a.c, l32, hh);
+        qk_tile<HD, KB, KPAD, true, kQlo>(Ks, qf, s, mb, c_sc, l32, hh, ql);
     };
     // s[kb][i] is key kt + 32*kb + 8*(i/4) + 4*hh + i%4 of query qrow.
     auto mask = [&](int kt) {
@@ -1320,6 +1305,18 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_pp_kernel(PrefillArgs a) 
     // ---- normalize and store: o[nb][i] is dim nb*32 + 8*(i/4) + 4*hh + i%4
     const float l_tot = l_run + shfl_xor(l_run, 32);
     if (!qvalid) return;
+    if (n_split > 1) {  // the split's partial, as in attn_prefill_kernel
+        const size_t row = ((size_t)sp * t + qrow) * a.H + h;
+        if (hh == 0) *reinterpret_cast<f32x2*>(a.part_ml + 2 * row) = f32x2{m_run, l_tot};
+        float* prow = a.part_o + row * HD;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4)
+                *reinterpret_cast<f32x4*>(prow + nb * 32 + 8 * g4 + 4 * hh) =
+                    f32x4{o[nb][4 * g4], o[nb][4 * g4 + 1], o[nb][4 * g4 + 2], o[nb][4 * g4 + 3]};
+        return;
+    }
     const float inv = 1.f / l_tot;
     float* orow = a.out + ((size_t)qrow * a.H + h) * HD;
     const float* grow = a.gate ? a.gate + ((size_t)qrow * a.H + h) * a.gate_stride : nullptr;
@@ -1336,13 +1333,13 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_pp_kernel(PrefillArgs a) 
 }
 
 // The ping-pong kernel takes 256 query rows per workgroup and one workgroup
-// per CU: it pays when there are at least two workgroups per CU (S >= 4096 at
-// 32 heads; at S = 2048 a single round of unequal causal workgroups leaves
-// CUs idle, and the 128-row kernel is faster).  LMX_PREFILL_KERNEL=pp|tile
-// forces one of them (tuning overrides, for tests and sweeps).  fp32 queries
-// take the 128-row kernel, which carries their f16 residual (qk_tile).
-static bool use_ping_pong(int hd, long n_tokens, long n_heads, lmx_dtype q_dt) {
-    if (hd != 128 || q_dt != LMX_F16) return false;
+// per CU.  f16 queries: it pays when there are at least two workgroups per CU
+// (S >= 4096 at 32 heads; at S = 2048 a single round of unequal causal
+// workgroups leaves CUs idle, and the 128-row kernel is faster).  fp32
+// queries: ping_pong_f32_splits.  LMX_PREFILL_KERNEL=pp|tile forces one of
+// them (tuning overrides, for tests and sweeps).
+static bool use_ping_pong(int hd, long n_tokens, long n_heads) {
+    if (hd != 128) return false;
     if (const int f = tuning().prefill_kernel; f >= 0) return f == 1;
     return (n_tokens + kPpBM - 1) / kPpBM * n_heads >= 512;
 }
@@ -1356,11 +1353,14 @@ static int prefill_gp(int G) {
 }
 
 // Key splits for attn_prefill_kernel and attn_prefill_wide_kernel.  When the
-// query tiles give fewer workgroups than the CUs hold at once (two per CU, one
-// of the wide kernel's), as for a short chunk on a long cache, each tile's key
-// range is cut into splits until that many are in flight, keeping at least
+// query tiles give fewer workgroups than the CUs hold at once (two per CU; one
+// of the wide kernel's, or of head_dim 128 with fp32 queries, whose residuals
+// take the LDS to 104 KB), as for a short chunk on a long cache, each tile's
+// key range is cut into splits until that many are in flight, keeping at least
 // kMinSplitTiles tiles of 64 keys per split (half as many in the wide kernel,
 // whose tiles cost four times the MFMAs a row); a merge kernel combines them.
+// (fp32 queries at 32 heads on 8, us a call with room for two counted and for
+// one: 1536 tokens 79 -> 55, 1800 tokens 103 -> 73.)
 constexpr int kMinSplitTiles = 8;
 constexpr int kMaxSplits = 16;
 constexpr int kCus = 256;
@@ -1370,15 +1370,59 @@ int prefill_wide_rows(int hd);
 int prefill_wide_gp(int G);
 lmx_status prefill_wide(const PrefillArgs& a, int hd, lmx_dtype q_dt, bool lin, hipStream_t st);
 
+// Estimated time of a head_dim 128 call with fp32 queries in us: workgroups of
+// bm rows, their key ranges cut into sp splits, tile_us per 64-key tile, one
+// workgroup a CU, heaviest first.  The longest unit bounds it from below, and
+// so does the CUs' mean load plus what the last round leaves idle of the
+// lightest unit.  A split costs its partials' trip through memory (written
+// and read back at 3 TB/s) and the merge launch, 8 us.
+static float f32_prefill_us(const lmx_attn_params* p, int bm, int sp, float tile_us) {
+    const int bn = 64;
+    const long t = p->n_tokens, end = (long)p->base_pos + t, w = p->window;
+    const long most = !w ? end : std::min<long>(end, p->bidi ? 2 * w - 1 : w);
+    const long units = (t + bm - 1) / bm * (long)p->n_heads * sp, rounds = (units + kCus - 1) / kCus;
+    const long longest = (std::min(end, most + bm) + bn - 1) / bn;
+    const long first = p->bidi ? longest : std::min<long>(longest, ((long)p->base_pos + bm + bn - 1) / bn);
+    const float load = 0.5f * (float)(first + longest) * (float)units / (float)sp / kCus +
+                       (float)(rounds * kCus - units) / kCus * (float)first / (float)sp;
+    const float tiles = std::max((float)((longest + sp - 1) / sp), load);
+    return tiles * tile_us + (sp > 1 ? 8.f + (float)t * (float)p->n_heads * 128.f * 8.f * (float)sp / 3e6f : 0.f);
+}
+
+// Key splits of the ping-pong kernel for fp32 queries, 0 where the 128-row
+// kernel is the faster one.  The residuals leave that kernel one wave per SIMD
+// (2.3 us a tile; the ping-pong kernel 2.7, for twice the rows, and 4 us more
+// before its first tile), so it pays wherever 256-row workgroups, cut into
+// splits if need be, spread as evenly over the CUs.  The five figures are
+// fitted to 56 calls (192 to 6000 tokens, at positions 0 to 4096, 16 and 32
+// heads); the kernel they choose is the faster one or within 5% of it.  At
+// 32 heads on 8, 128-row kernel : ping-pong, us a call: 512 tokens 25 : 32,
+// 2048 81 : 87, 3000 171 : 130, 4000 273 : 204; 512 tokens at position 4096
+// 83 : 73, 2048 there 314 : 264.
+static int ping_pong_f32_splits(const lmx_attn_params* p, int tile_splits) {
+    const int forced = tuning().prefill_kernel;
+    if (p->head_dim != 128 || forced == 0) return 0;
+    int best = 0;
+    float best_us = forced == 1 ? 3.4e38f : f32_prefill_us(p, kPfBM, tile_splits, 2.3f);
+    const long longest = ((long)p->base_pos + p->n_tokens) / 64;
+    for (int sp = 1; sp <= kMaxSplits && (sp == 1 || longest >= 4 * sp); ++sp) {
+        const float us = 4.f + f32_prefill_us(p, kPpBM, sp, 2.7f);
+        if (us < best_us) {
+            best = sp;
+            best_us = us;
+        }
+    }
+    return best;
+}
+
 static int prefill_splits(const lmx_attn_params* p, lmx_dtype q_dt) {
     const int hd = (int)p->head_dim;
-    if (use_ping_pong(hd, (long)p->n_tokens, (long)p->n_heads, q_dt)) return 1;
     const bool wide = hd >= 256;
     const int G = (int)(p->n_heads / p->n_kv_heads);
     const int gp = wide ? prefill_wide_gp(G) : prefill_gp(G);
     const long bm = wide ? prefill_wide_rows(hd) / gp : kPfBM / gp;
     const long n_wg = (long)((p->n_tokens + bm - 1) / bm) * (p->n_heads / gp);
-    const long slots = (long)kCus * (wide ? 1 : 2);
+    const long slots = (long)kCus * (wide || (hd == 128 && q_dt != LMX_F16) ? 1 : 2);
     if (n_wg >= slots) return 1;
     const int bn = 64;
     // the longest key range a workgroup covers: one query's range plus the
@@ -1393,11 +1437,23 @@ static int prefill_splits(const lmx_attn_params* p, lmx_dtype q_dt) {
 
 static size_t round_up256(size_t x) { return (x + 255) / 256 * 256; }
 
-size_t prefill_workspace_bytes(const lmx_attn_params* p) {
-    const int sp = std::max(prefill_splits(p, LMX_F16), prefill_splits(p, LMX_F32));
+static size_t split_bytes(const lmx_attn_params* p, int sp) {
     if (sp == 1) return 0;
     const size_t rows = (size_t)sp * p->n_tokens * p->n_heads;
     return round_up256(rows * 2 * sizeof(float)) + round_up256(rows * p->head_dim * sizeof(float));
+}
+
+// The workspace without which a call is refused: the 128-row kernel's (f16
+// ping-pong calls are not split).  A ping-pong call with fp32 queries can use
+// more (prefill_workspace_bytes) and goes to the 128-row kernel in less.
+size_t prefill_needed_bytes(const lmx_attn_params* p) {
+    if (use_ping_pong((int)p->head_dim, (long)p->n_tokens, (long)p->n_heads)) return split_bytes(p, prefill_splits(p, LMX_F32));
+    return split_bytes(p, std::max(prefill_splits(p, LMX_F16), prefill_splits(p, LMX_F32)));
+}
+
+size_t prefill_workspace_bytes(const lmx_attn_params* p) {
+    const int sp = ping_pong_f32_splits(p, prefill_splits(p, LMX_F32));
+    return std::max(prefill_needed_bytes(p), split_bytes(p, std::max(sp, 1)));
 }
 
 bool prefill_supported(const lmx_attn_params* p, lmx_dtype q_dt) {
@@ -1409,10 +1465,18 @@ lmx_status prefill_fwd(const lmx_attn_params* p, const AttnIo& io, const void* q
                        const void* k_cache, const void* v_cache, const void* k_cur, const void* v_cur,
                        float* out, void* ws, size_t ws_bytes, hipStream_t st) {
     PrefillArgs a{};
-    a.n_split = prefill_splits(p, q_dt);
-    if (a.n_split > 1) {
-        if (!ws || ws_bytes < prefill_workspace_bytes(p)) return LMX_E_WORKSPACE;
+    bool pp = q_dt == LMX_F16 && use_ping_pong((int)p->head_dim, (long)p->n_tokens, (long)p->n_heads);
+    a.n_split = pp ? 1 : prefill_splits(p, q_dt);
+    if (const size_t need = pp ? 0 : prefill_needed_bytes(p)) {
+        if (!ws || ws_bytes < need) return LMX_E_WORKSPACE;
         if (((uintptr_t)ws & 255) != 0) return LMX_E_ALIGN;
+    }
+    if (q_dt != LMX_F16) {
+        const int sp = ping_pong_f32_splits(p, a.n_split);
+        pp = sp == 1 || (sp > 1 && ws && ((uintptr_t)ws & 255) == 0 && ws_bytes >= split_bytes(p, sp));
+        if (pp) a.n_split = sp;
+    }
+    if (a.n_split > 1) {
         const size_t rows = (size_t)a.n_split * p->n_tokens * p->n_heads;
         a.part_ml = static_cast<float*>(ws);
         a.part_o = reinterpret_cast<float*>(static_cast<char*>(ws) + round_up256(rows * 2 * sizeof(float)));
@@ -1437,7 +1501,6 @@ lmx_status prefill_fwd(const lmx_attn_params* p, const AttnIo& io, const void* q
     a.c = p->scale * kLog2e;
     window_magic((uint32_t)a.window, &a.w_magic, &a.w_shift);
     const int hd = (int)p->head_dim;
-    const bool pp = use_ping_pong(hd, (long)p->n_tokens, (long)p->n_heads, q_dt);
     const bool wide = hd >= 256;
     a.gp = wide ? prefill_wide_gp(a.G) : prefill_gp(a.G);
     const int bm = wide ? prefill_wide_rows(hd) / a.gp : pp ? kPpBM / a.gp : kPfBM / a.gp;
@@ -1480,8 +1543,9 @@ lmx_status prefill_fwd(const lmx_attn_params* p, const AttnIo& io, const void* q
     } else if (kh) {  // f16 queries only
         if (hd == 64) hipLaunchKernelGGL((attn_prefill_kh_kernel<f16, 64>), grid, dim3(256), 0, st, a);
         else hipLaunchKernelGGL((attn_prefill_kh_kernel<f16, 128>), grid, dim3(256), 0, st, a);
-    } else if (pp) {  // f16 queries only
-        LMX_PP(f16);
+    } else if (pp) {
+        if (q_dt == LMX_F16) LMX_PP(f16);
+        else LMX_PP(float);
     } else if (q_dt == LMX_F16) {
         if (hd == 64) LMX_PF(f16, 64);
         else if (hd == 128) LMX_PF(f16, 128);

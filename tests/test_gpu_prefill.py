@@ -5,6 +5,7 @@ Full-size cases (S=8192) are checked on a seeded sample of query rows: a
 query's causal output depends only on its own position and the keys it sees,
 so the oracle run at t=1 for that position is the same computation.
 """
+import ctypes
 import sys
 
 import numpy as np
@@ -94,6 +95,41 @@ def test_chunked_prefill_512_onto_4096():
 def test_f32_query_prefill():
     c = AttnCase(77, t=300, H=16, Hkv=4, hd=128, n_pos=700)
     check(c, base=400)
+
+
+@pytest.mark.parametrize("t,base,window,bidi", [
+    (192, 0, 0, False), (255, 1, 0, False), (257, 63, 0, False),  # edges of 256-row tiles
+    (600, 1500, 0, False), (257, 5000, 0, False),                 # key splits, some of them empty for the first rows
+    (700, 1000, 0, True),                                         # every row sees every split
+    (300, 900, 150, False), (513, 40, 700, False)])               # rings, the batch's own rows beside them
+def test_f32_query_key_splits(t, base, window, bidi):
+    """fp32 queries carry their f16 residual through either kernel, in one
+    pass over the keys or in splits of them that a merge combines."""
+    c = AttnCase(t + base, t=t, H=8, Hkv=2, hd=128, n_pos=base + t, qk_norm=True)
+    check(c, base=base, window=window, bidi=bidi, ring=window > 0, k_cur=window > 0, scale=1.0 if window else None)
+
+
+def test_f32_query_without_the_splits_workspace(tuning_env):
+    """A call that needs no workspace but can use one for key splits (256-row
+    workgroups 1.1 times the CUs) runs on the tile kernel when given none."""
+    t, H, Hkv, base = 1920, 35, 5, 4096
+    c = AttnCase(2049, t=t, H=H, Hkv=Hkv, hd=128, n_pos=base + t, qk_norm=True)
+    q, k, v = dev(c.q), dev(c.k16, torch.float16), dev(c.v16, torch.float16)
+    p = lmx.attn_params(n_tokens=t, n_heads=H, n_kv_heads=Hkv, head_dim=128, base_pos=base, n_slots=base + t)
+    offered = lmx.lib().lmx_attn_workspace_bytes(ctypes.byref(p))
+    assert (offered > 0) == (lmx_kernel() == "pp")
+    outs = []
+    for forced in (None, "tile"):
+        if forced:
+            tuning_env("LMX_PREFILL_KERNEL", forced)
+        out = torch.empty_like(q)
+        rc = lmx.lib().lmx_attn_fwd(ctypes.byref(p), q.data_ptr(), lmx.F32, k.data_ptr(), v.data_ptr(), lmx.F16,
+                                    None, None, out.data_ptr(), None, 0,
+                                    torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        torch.cuda.synchronize()
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1])
 
 
 @pytest.mark.parametrize("H,Hkv,hd", [(8, 8, 64), (16, 2, 64), (16, 8, 256), (24, 4, 128)])
