@@ -285,10 +285,14 @@ def _ptr(t) -> Optional[int]:
 
 
 def _stream(stream) -> Optional[int]:
+    if stream is not None:
+        return stream.cuda_stream
     torch = _torch()
-    if stream is None:
-        stream = torch.cuda.current_stream()
-    return stream.cuda_stream
+    if not torch.cuda.is_initialized():
+        return torch.cuda.current_stream().cuda_stream
+    # the raw handle alone: a call of a few microseconds notices the
+    # torch.cuda.Stream object that current_stream() makes for it
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _dt(t) -> int:
