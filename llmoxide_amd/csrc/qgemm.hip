@@ -336,6 +336,7 @@ __global__ __launch_bounds__(512, 1) void qgemm_kernel(GemmArgs a) {
     __shared__ __attribute__((aligned(16))) f16 xs_s[2][OFFSET ? TM * 16 : 8];  // x sums / 16: 8 hi, 8 lo
     __shared__ __attribute__((aligned(16))) float rs_s[2][TM];  // a token's scale ratio of this chunk
     __shared__ __attribute__((aligned(16))) int chg_s[2][8];    // per staging wave: some ratio is not 1
+    __shared__ int k_s[TM];  // a token's scale exponent after the last chunk
     auto xh = [&](int b) { return reinterpret_cast<f16*>(xy_s) + b * 2 * XB; };
     auto xl = [&](int b) { return xh(b) + XB; };
 
@@ -371,9 +372,12 @@ __global__ __launch_bounds__(512, 1) void qgemm_kernel(GemmArgs a) {
     };
     // ---- x: token wave * NX + u, floats 4 lane .. + 3 of the chunk
     f32x4 rx[NX];
-    int kx[NX];  // running scale exponents (100: no nonzero x yet)
+    // running scale exponents; kNone, which no chunk's bound reaches (the
+    // smallest denormal's is 14 + 148): no nonzero x yet
+    constexpr int kNone = 1000;
+    int kx[NX];
 #pragma unroll
-    for (int u = 0; u < NX; ++u) kx[u] = 100;
+    for (int u = 0; u < NX; ++u) kx[u] = kNone;
     auto load_x = [&](int ch) __attribute__((always_inline)) {
         const int k = ch * kGK + 4 * lane;
 #pragma unroll
@@ -432,7 +436,10 @@ __global__ __launch_bounds__(512, 1) void qgemm_kernel(GemmArgs a) {
                 int kn = kx[u];
                 if (m > 0.f && m <= 3.402823466e38f)
                     kn = min(kn, m >= 0.015625f && m < 16384.f ? 0 : 14 - __builtin_amdgcn_frexp_expf(m));
-                const float ratio = kx[u] == 100 ? 1.f : __builtin_amdgcn_ldexpf(1.f, kn - kx[u]);
+                // (y is 0 or not finite before the first nonzero x; a ratio
+                // below 2^-126 leaves nothing of a finite y, and must not be 0
+                // beside an infinite one)
+                const float ratio = kx[u] == kNone ? 1.f : __builtin_amdgcn_ldexpf(1.f, max(kn - kx[u], -126));
                 kx[u] = kn;
                 changed |= ratio != 1.f;
                 plain = plain && kn == 0;
@@ -583,7 +590,7 @@ __global__ __launch_bounds__(512, 1) void qgemm_kernel(GemmArgs a) {
     }
 
     // ---- the KQ partial sums, [range][token][row], through the x buffers;
-    // each staging wave knows its tokens' final scales
+    // each staging wave knows its tokens' final exponents
     __syncthreads();
     float* y_s = reinterpret_cast<float*>(xy_s);
 #pragma unroll
@@ -597,7 +604,7 @@ __global__ __launch_bounds__(512, 1) void qgemm_kernel(GemmArgs a) {
             }
     if (lane == 0)
 #pragma unroll
-        for (int u = 0; u < NX; ++u) rs_s[0][wave * NX + u] = kx[u] == 100 ? 1.f : __builtin_amdgcn_ldexpf(1.f, -kx[u]);
+        for (int u = 0; u < NX; ++u) k_s[wave * NX + u] = kx[u] == kNone ? 0 : kx[u];
     __syncthreads();
 #pragma unroll
     for (int i = tid; i < TM * TN; i += 512) {
@@ -606,7 +613,7 @@ __global__ __launch_bounds__(512, 1) void qgemm_kernel(GemmArgs a) {
         float v = y_s[i];
 #pragma unroll
         for (int q = 1; q < KQ; ++q) v += y_s[q * TM * TN + i];
-        a.y[(size_t)(t0 + tok) * a.rows + r0 + row] = v * rs_s[0][tok];
+        a.y[(size_t)(t0 + tok) * a.rows + r0 + row] = __builtin_amdgcn_ldexpf(v, -k_s[tok]);
     }
 }
 

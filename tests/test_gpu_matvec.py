@@ -201,3 +201,37 @@ def test_gemm_bf16_weight_range():
     got, ref = y.cpu().numpy().astype(np.float64), x.astype(np.float64) @ w64.T
     for r in range(rows):  # each row against its own scale
         assert np.abs(got[:, r] - ref[:, r]).max() <= 3e-6 * np.abs(ref[:, r]).max(), r
+
+
+def f64_ref(name, w, rows, in_dim, x):
+    """W x in float64 (W as the format's exact values)."""
+    W = oracle.dequant(oracle.QTYPES[name], w, rows * in_dim).reshape(rows, in_dim)
+    return x.astype(np.float64) @ W.astype(np.float64).T
+
+
+def gemm(name, w, rows, in_dim, x):
+    y = lmx.matvec(torch.from_numpy(w).cuda(), torch.from_numpy(x).cuda(), qtype=name, rows=rows, in_dim=in_dim)
+    torch.cuda.synchronize()
+    return y.cpu().numpy()
+
+
+@pytest.mark.parametrize("name", GEMM_TYPES + ["f16", "bf16"])
+@pytest.mark.parametrize("n_tok", [21, 49])
+def test_gemm_smallest_x(name, n_tok):
+    # x whose scale exponent is beyond 100 (below 2^-86), alone, before and
+    # after ordinary chunks and zero ones; the x stay normal floats
+    rows, in_dim = 70, 1024
+    say(f"gemm {name} smallest x n_tok={n_tok}")
+    w = oracle.quant_weights(oracle.QTYPES[name], rows, in_dim, 84)
+    x = oracle.normal(85, (n_tok, in_dim)).astype(np.float64)
+    ends = {0: (1e-30, 1e-30), 1: (1e-27, 1.0), 2: (1.0, 1e-27), 3: (0.0, 1e-30), 4: (1e-30, 0.0),
+            5: (1e-35, 1e-20), 6: (1.5 * 2.0 ** -86, 1e4)}
+    for t in range(n_tok):
+        first, rest = ends[t % 7]
+        x[t, :256] *= first
+        x[t, 256:] *= rest
+    x = x.astype(np.float32)
+    got, ref = gemm(name, w, rows, in_dim, x), f64_ref(name, w, rows, in_dim, x)
+    for t in range(n_tok):
+        err, scale = np.abs(got[t] - ref[t]).max(), np.abs(ref[t]).max()
+        assert err <= 3e-5 * scale, f"{name} token {t} (kind {t % 7}): max err {err} vs max |ref| {scale}"
