@@ -12,28 +12,30 @@
 //     Q4_K  q in [0, 15],     s = d * sc_g, o = -dmin * m_g  (groups of 32)
 //     Q6_K  q in [-32, 31],   s = d * sc_g, o = 0            (groups of 16)
 //     Q8_0  q in [-128, 127], s = d,        o = 0            (groups of 32)
-//   x is split into f16 x_hi + x_lo (|x - x_hi - x_lo| <= 2^-22 |x|), and all
-//   products run on v_mfma_f32_32x32x16_f16 with fp32 accumulation.  The
+//   x, scaled (below), is split into f16 x_hi + x_lo, and all products run on
+//   v_mfma_f32_32x32x16_f16 with fp32 accumulation.  The
 //   integer scales go into the weight operand, where the vector unit pays for
 //   them once a weight instead of once a token: sc_g q of Q4_K is at most 945
 //   and exact in f16; of Q6_K it is at most 4096 and exact as f16(sc_g q) plus
 //   a remainder (third product: remainder times x_hi).  Only d, one a
 //   super-block of 256, is applied to the fp32 sums (of a bf16 row, the power
 //   of two that brought 256 / KQ of its weights into f16's range).  Q4_K's offsets are one
-//   more MFMA a super-block: the m_g against the group sums of x (hi and lo,
-//   scaled by 1/16 into f16's range).  Q8_0's d has 11 bits of its own, so its
+//   more MFMA a super-block: the m_g against the group sums of the scaled x
+//   (hi and lo, times 1/16: at most 2^15).  Q8_0's d has 11 bits of its own, so its
 //   group sums are scaled in fp32.
 //
 //   Range: before the split, each token's x is multiplied by a power of two
-//   2^k_t (exact).  k_t is the running minimum over the chunks of a bound
-//   k_c: 0 while the token's largest |x| in the chunk lies in [2^-6, 2^14),
-//   else the k that brings it into [2^13, 2^14).  So no scaled value comes
-//   near f16's 65504, and a token whose x are all tiny is scaled up instead
-//   of falling into f16 subnormals.  Every partial sum of a token is in one
-//   scaled domain: when a chunk lowers k_t, the token's accumulated y is
-//   first multiplied by the (exact) ratio, and the store multiplies by
-//   2^-k_t.  Elements far below their chunk's maximum keep an absolute error
-//   of about 2^-22 of the largest value met, as fp32 summation would.
+//   2^k_t (exact).  Its first nonzero chunk sets k_t so that the chunk's
+//   largest |x| lands in [2^11, 2^12); a later chunk whose scaled |x| reach
+//   2^14 lowers it to do the same.  So no scaled value comes near f16's 65504,
+//   and |x - x_hi - x_lo| is at most 2^-22 |x| for every x down to 2^-14 of
+//   the largest met, and 2^-36 of that largest below: f16's subnormals begin
+//   at 2^-14, so a residual keeps its 11 bits only from a scaled |x| of 2^-3
+//   up.  (Left unscaled, x of rms 0.006 cost 2.9e-6 of the result, 0.1 2.1e-7;
+//   the matvec costs 1.0e-7 to 2.7e-7, this 1.2e-7 to 1.9e-7 at any rms.)  Every
+//   partial sum of a token is in one scaled domain: when a chunk lowers k_t,
+//   the token's accumulated y is first multiplied by the (exact) ratio, and
+//   the store multiplies by 2^-k_t.
 //
 // A workgroup of eight waves owns 32 TT tokens x 32 RT WR rows and walks K in
 // chunks of 256.  x goes through LDS, two buffers of swizzled f16 hi / lo
@@ -372,8 +374,8 @@ __global__ __launch_bounds__(512, 1) void qgemm_kernel(GemmArgs a) {
     };
     // ---- x: token wave * NX + u, floats 4 lane .. + 3 of the chunk
     f32x4 rx[NX];
-    // running scale exponents; kNone, which no chunk's bound reaches (the
-    // smallest denormal's is 14 + 148): no nonzero x yet
+    // running scale exponents; kNone, which no chunk sets (the smallest
+    // denormal sets 12 + 148): no nonzero x yet
     constexpr int kNone = 1000;
     int kx[NX];
 #pragma unroll
@@ -387,8 +389,7 @@ __global__ __launch_bounds__(512, 1) void qgemm_kernel(GemmArgs a) {
             rx[u] = *reinterpret_cast<const f32x4*>(a.x + (size_t)tok * a.in_dim + min(k, a.in_dim - 4));
         }
     };
-    int ones = 0;        // bit b: buffer b's ratios of this wave's tokens are 1 (uniform)
-    bool plain = false;  // every k_t of this wave's tokens is 0 (uniform)
+    int ones = 0;  // bit b: buffer b's ratios of this wave's tokens are 1 (uniform)
     // One token's floats to hi / lo rows, and (Q4_K) its group sums.
     auto emit = [&](int b, int u, const f32x4& v) __attribute__((always_inline)) {
         const int tok = wave * NX + u;
@@ -416,12 +417,20 @@ __global__ __launch_bounds__(512, 1) void qgemm_kernel(GemmArgs a) {
 #pragma unroll
             for (int u = 0; u < NX; ++u) rx[u] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
-        // once every k_t is 0 and no |x| reaches 2^14, nothing changes (a NaN
-        // passes through as it is)
+        // nothing changes while no scaled |x| reaches 2^14 (a NaN passes through
+        // as it is; before a token's first nonzero x its scale takes any to inf)
+        f32x4 v[NX];
         float top = 0.f;
+        auto scale = [&](int u) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < NX; ++u) top = absmax3(rx[u][2], rx[u][3], absmax3(rx[u][0], rx[u][1], top));
-        if (plain && __builtin_amdgcn_ballot_w64(top >= 16384.f) == 0) {
+            for (int j = 0; j < 4; ++j) v[u][j] = __builtin_amdgcn_ldexpf(rx[u][j], kx[u]);
+        };
+#pragma unroll
+        for (int u = 0; u < NX; ++u) {
+            scale(u);
+            top = absmax3(v[u][2], v[u][3], absmax3(v[u][0], v[u][1], top));
+        }
+        if (__builtin_amdgcn_ballot_w64(top >= 16384.f) == 0) {
             if (!(ones >> b & 1)) {
                 if (lane < NX) rs_s[b][wave * NX + lane] = 1.f;
                 if (lane == 0) chg_s[b][wave] = 0;
@@ -429,32 +438,26 @@ __global__ __launch_bounds__(512, 1) void qgemm_kernel(GemmArgs a) {
             }
         } else {
             int changed = 0;
-            plain = true;
 #pragma unroll
             for (int u = 0; u < NX; ++u) {
                 const float m = wave_max64(absmax3(rx[u][2], rx[u][3], absmax3(rx[u][0], rx[u][1], 0.f)));
                 int kn = kx[u];
-                if (m > 0.f && m <= 3.402823466e38f)
-                    kn = min(kn, m >= 0.015625f && m < 16384.f ? 0 : 14 - __builtin_amdgcn_frexp_expf(m));
+                if (m > 0.f && m <= 3.402823466e38f && __builtin_amdgcn_ldexpf(m, kn) >= 16384.f)
+                    kn = 12 - __builtin_amdgcn_frexp_expf(m);
                 // (y is 0 or not finite before the first nonzero x; a ratio
                 // below 2^-126 leaves nothing of a finite y, and must not be 0
                 // beside an infinite one)
                 const float ratio = kx[u] == kNone ? 1.f : __builtin_amdgcn_ldexpf(1.f, max(kn - kx[u], -126));
                 kx[u] = kn;
                 changed |= ratio != 1.f;
-                plain = plain && kn == 0;
                 if (lane == 0) rs_s[b][wave * NX + u] = ratio;
+                scale(u);
             }
             if (lane == 0) chg_s[b][wave] = changed;
             ones &= ~(1 << b);
         }
 #pragma unroll
-        for (int u = 0; u < NX; ++u) {
-            f32x4 v;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) v[j] = __builtin_amdgcn_ldexpf(rx[u][j], kx[u]);
-            emit(b, u, v);
-        }
+        for (int u = 0; u < NX; ++u) emit(b, u, v[u]);
     };
 
     f32x16 y[TT][RT];

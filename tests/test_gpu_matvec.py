@@ -235,3 +235,20 @@ def test_gemm_smallest_x(name, n_tok):
     for t in range(n_tok):
         err, scale = np.abs(got[t] - ref[t]).max(), np.abs(ref[t]).max()
         assert err <= 3e-5 * scale, f"{name} token {t} (kind {t % 7}): max err {err} vs max |ref| {scale}"
+
+
+@pytest.mark.parametrize("name", GEMM_TYPES + ["f16", "bf16"])
+@pytest.mark.parametrize("n_tok", [20, 70])
+def test_gemm_small_x_keeps_its_bits(name, n_tok):
+    # the split of x into two f16 parts costs no more at an attention or FFN
+    # output's scale than at 1.  Bound: 2^-21 of the result's 2-norm, eight
+    # fp32 roundings, for the fp32 sums of 2048 products and 8 to 64 blocks.
+    rows, in_dim = 200, 2048
+    w = oracle.quant_weights(oracle.QTYPES[name], rows, in_dim, 86)
+    x0 = oracle.normal(87, (n_tok, in_dim))
+    for rms in (1.0, 0.1, 0.02, 0.006, 3e-5):
+        x = x0 * np.float32(rms)
+        got, ref = gemm(name, w, rows, in_dim, x), f64_ref(name, w, rows, in_dim, x)
+        err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+        say(f"gemm {name} n_tok={n_tok} x rms {rms}: {err:.2e}")
+        assert err <= 2.0 ** -21, (name, rms, err)
