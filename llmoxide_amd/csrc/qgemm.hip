@@ -35,7 +35,7 @@
 //   the matvec costs 1.0e-7 to 2.7e-7, this 1.2e-7 to 1.9e-7 at any rms.)  Every
 //   partial sum of a token is in one scaled domain: when a chunk lowers k_t,
 //   the token's accumulated y is first multiplied by the (exact) ratio, and
-//   the store multiplies by 2^-k_t.
+//   the store multiplies by 2^-k_t.  Infinities: see qgemm_kernel.
 //
 // A workgroup of eight waves owns 32 TT tokens x 32 RT WR rows and walks K in
 // chunks of 256.  x goes through LDS, two buffers of swizzled f16 hi / lo
@@ -66,6 +66,8 @@ namespace lmx {
 enum GType { kGF16 = 1, kGQ8_0 = 8, kGQ4K = 12, kGQ6K = 14, kGBF16 = 30 };
 template <int TY>
 constexpr bool g_dense() { return TY == kGF16 || TY == kGBF16; }
+
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kGK = 256;  // k per chunk: a K-quant super-block, eight Q8_0 blocks
 
@@ -134,6 +136,12 @@ __device__ __forceinline__ void bytes_1024(uint32_t q, f16x2& a, f16x2& b) {
     b = as_h2(((q >> 8) & 0x00FF00FFu) | 0x64006400u);
 }
 __device__ __forceinline__ f16x2 pk_fma(f16x2 a, f16x2 b, f16x2 c) { return __builtin_elementwise_fma(a, b, c); }
+
+// An infinity or NaN as +-65504.
+__device__ __forceinline__ f16x2 finite2(f16x2 x) {
+    const f16x2 hi = {(f16)65504.f, (f16)65504.f}, lo = {(f16)-65504.f, (f16)-65504.f};
+    return __builtin_elementwise_min(__builtin_elementwise_max(x, lo), hi);
+}
 
 // A wave's share of a chunk of one weight row: its raw bytes, read from LDS
 // once, and the operand of each of its k-steps.  KQ ranges a chunk; lane half
@@ -269,8 +277,8 @@ struct WFrag<kGQ8_0, KQ> {
 };
 
 // Dense rows: range = 256 / KQ consecutive weights.  bf16 becomes f16 times a
-// power of two that brings the range's largest weight into [2^14, 2^15): exact
-// for weights down to 2^-31 of it, 2^-39 of it below.
+// power of two that brings the range's largest finite weight into [2^14, 2^15):
+// exact for weights down to 2^-31 of it, 2^-39 of it below.
 template <int TY, int KQ>
 struct DFrag {
     static constexpr int NK = 16 / KQ;
@@ -279,22 +287,34 @@ struct DFrag {
     __device__ static __forceinline__ int k_of(int s, int kq, int hh) { return 16 * (NK * kq + s) + 8 * hh; }
     // left: weights of the chunk that lie inside the row
     __device__ __forceinline__ void load(const uint8_t* row, int kq, int hh, int left) {
-        uint32_t top = 0;
+        u16x2 top = {0, 0};  // largest magnitudes (bit patterns order as their values)
 #pragma unroll
         for (int s = 0; s < NK; ++s) {
             const int k = k_of(s, kq, hh);
             raw[s] = k < left ? *reinterpret_cast<const uint4*>(row + 2 * k) : uint4{0u, 0u, 0u, 0u};
-            if constexpr (TY == kGBF16) {
+        }
+        auto each = [&](auto f) __attribute__((always_inline)) {
+#pragma unroll
+            for (int s = 0; s < NK; ++s) {
                 const uint32_t w[4] = {raw[s].x, raw[s].y, raw[s].z, raw[s].w};
 #pragma unroll
-                for (int i = 0; i < 4; ++i) top = max(top, max(w[i] & 0x7FFF0000u, (w[i] << 16) & 0x7FFF0000u));
+                for (int i = 0; i < 4; ++i) f(__builtin_bit_cast(u16x2, w[i] & 0x7FFF7FFFu));
             }
-        }
+        };
         sc = 0;
         if constexpr (TY == kGBF16) {
-            const float t = __builtin_bit_cast(float, top);
-            const float m = fmaxf(t, shfl_xor(t, 32));  // (every bit pattern orders as its float)
-            if (m > 0.f && m <= 3.402823466e38f) sc = 15 - __builtin_amdgcn_frexp_expf(m);
+            each([&](u16x2 m) { top = __builtin_elementwise_max(top, m); });
+            constexpr uint16_t inf = 0x7F80;
+            if (__builtin_amdgcn_ballot_w64(max(top[0], top[1]) >= inf)) {  // the largest finite one, then
+                top = u16x2{0, 0};
+                each([&](u16x2 m) {
+                    const u16x2 fin = {m[0] < inf ? m[0] : (uint16_t)0, m[1] < inf ? m[1] : (uint16_t)0};
+                    top = __builtin_elementwise_max(top, fin);
+                });
+            }
+            const float t = __builtin_bit_cast(float, (uint32_t)max(top[0], top[1]) << 16);
+            const float m = fmaxf(t, shfl_xor(t, 32));
+            if (m > 0.f) sc = 15 - __builtin_amdgcn_frexp_expf(m);
         }
     }
     __device__ __forceinline__ f16x8 step(int s) const {
@@ -323,22 +343,37 @@ template <int KQ>
 struct WFrag<kGBF16, KQ> : DFrag<kGBF16, KQ> {};
 
 template <int TY, int TT, int RT, int WR>
-__global__ __launch_bounds__(512, 1) void qgemm_kernel(GemmArgs a) {
+struct GemmLds {
+    static constexpr int TM = 32 * TT, TN = 32 * RT * WR, KQ = 8 / WR;
+    // x rows of 256 halfs, 16-byte pieces XORed with the row, hi and lo of two
+    // chunks; also the partial sums at the end
+    static constexpr int XB = TM * kGK;
+    static constexpr int X = 2 * 2 * XB * 2, Y = KQ * TM * TN * 4;
+    alignas(16) unsigned char xy[X > Y ? X : Y];
+    alignas(16) unsigned char w[TN * GTraits<TY>::stride * 16 + 16];
+    alignas(16) f16 xs[2][TY == kGQ4K ? TM * 16 : 8];  // x sums / 16: 8 hi, 8 lo
+    alignas(16) float rs[2][TM];  // a token's scale ratio of this chunk
+    alignas(16) int chg[2][8];    // per staging wave: some ratio is not 1
+    int k[TM];  // a token's scale exponent after the last chunk
+    int nan;    // some result is NaN
+};
+
+// INF: dense rows, with infinite x and weights kept apart from the split's 0
+// (see qgemm_kernel).
+template <int TY, int TT, int RT, int WR, bool INF>
+__device__ __forceinline__ void qgemm_tile(const GemmArgs& a, GemmLds<TY, TT, RT, WR>& lds) {
     constexpr int TM = 32 * TT, TN = 32 * RT * WR, KQ = 8 / WR;
     constexpr int NK = 16 / KQ;  // k-steps of a wave per chunk
     constexpr int STR = GTraits<TY>::stride * 16, PC = GTraits<TY>::stride, NPC = GTraits<TY>::pieces;
     constexpr int NX = TM / 8;   // tokens a wave stages per chunk
     constexpr bool OFFSET = TY == kGQ4K;
-    // x rows of 256 halfs, 16-byte pieces XORed with the row; also the
-    // partial sums at the end
     constexpr int XB = TM * kGK;
-    constexpr int SMEM_X = 2 * 2 * XB * 2, SMEM_Y = KQ * TM * TN * 4;
-    __shared__ __attribute__((aligned(16))) unsigned char xy_s[SMEM_X > SMEM_Y ? SMEM_X : SMEM_Y];
-    __shared__ __attribute__((aligned(16))) unsigned char w_s[TN * STR + 16];
-    __shared__ __attribute__((aligned(16))) f16 xs_s[2][OFFSET ? TM * 16 : 8];  // x sums / 16: 8 hi, 8 lo
-    __shared__ __attribute__((aligned(16))) float rs_s[2][TM];  // a token's scale ratio of this chunk
-    __shared__ __attribute__((aligned(16))) int chg_s[2][8];    // per staging wave: some ratio is not 1
-    __shared__ int k_s[TM];  // a token's scale exponent after the last chunk
+    auto& xy_s = lds.xy;
+    auto& w_s = lds.w;
+    auto& xs_s = lds.xs;
+    auto& rs_s = lds.rs;
+    auto& chg_s = lds.chg;
+    auto& k_s = lds.k;
     auto xh = [&](int b) { return reinterpret_cast<f16*>(xy_s) + b * 2 * XB; };
     auto xl = [&](int b) { return xh(b) + XB; };
 
@@ -396,6 +431,7 @@ __global__ __launch_bounds__(512, 1) void qgemm_kernel(GemmArgs a) {
         // hi once (pinned: the residual is taken against these very
         // registers); in the order 0 2 1 3
         f16x2 h0 = {(f16)v[0], (f16)v[2]}, h1 = {(f16)v[1], (f16)v[3]};
+        if constexpr (INF) h0 = finite2(h0), h1 = finite2(h1);  // an infinite x: all residual (inf - inf is NaN)
         asm("" : "+v"(h0), "+v"(h1));
         const f16x4 hi = {h0[0], h0[1], h1[0], h1[1]};
         const f16x4 lo = {(f16)(v[0] - (float)h0[0]), (f16)(v[2] - (float)h0[1]), (f16)(v[1] - (float)h1[0]),
@@ -440,9 +476,15 @@ __global__ __launch_bounds__(512, 1) void qgemm_kernel(GemmArgs a) {
             int changed = 0;
 #pragma unroll
             for (int u = 0; u < NX; ++u) {
-                const float m = wave_max64(absmax3(rx[u][2], rx[u][3], absmax3(rx[u][0], rx[u][1], 0.f)));
+                float m = wave_max64(absmax3(rx[u][2], rx[u][3], absmax3(rx[u][0], rx[u][1], 0.f)));
+                if (m > 3.402823466e38f) {  // (uniform) the largest finite one, then
+                    m = 0.f;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) m = fmaxf(m, fabsf(rx[u][j]) <= 3.402823466e38f ? fabsf(rx[u][j]) : 0.f);
+                    m = wave_max64(m);
+                }
                 int kn = kx[u];
-                if (m > 0.f && m <= 3.402823466e38f && __builtin_amdgcn_ldexpf(m, kn) >= 16384.f)
+                if (m > 0.f && __builtin_amdgcn_ldexpf(m, kn) >= 16384.f)
                     kn = 12 - __builtin_amdgcn_frexp_expf(m);
                 // (y is 0 or not finite before the first nonzero x; a ratio
                 // below 2^-126 leaves nothing of a finite y, and must not be 0
@@ -534,14 +576,22 @@ __global__ __launch_bounds__(512, 1) void qgemm_kernel(GemmArgs a) {
             }
 #pragma unroll
             for (int n = 0; n < RT; ++n) {
-                f16x8 q, ql;
+                f16x8 q, ql, qf;  // qf: beside x_lo
                 if constexpr (TY == kGQ6K) w[n].step(s, kq, q, ql);
                 else if constexpr (TY == kGQ4K) q = w[n].step(s, kq);
                 else q = w[n].step(s);
+                qf = q;
+                if constexpr (INF)
+#pragma unroll
+                    for (int i = 0; i < 8; i += 2) {
+                        const f16x2 f = finite2(f16x2{q[i], q[i + 1]});
+                        qf[i] = f[0];
+                        qf[i + 1] = f[1];
+                    }
 #pragma unroll
                 for (int i = 0; i < TT; ++i) {
                     acc[i][n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], q, acc[i][n], 0, 0, 0);
-                    acc[i][n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[i], q, acc[i][n], 0, 0, 0);
+                    acc[i][n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[i], qf, acc[i][n], 0, 0, 0);
                     if constexpr (TY == kGQ6K)
                         acc[i][n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], ql, acc[i][n], 0, 0, 0);
                 }
@@ -608,6 +658,7 @@ __global__ __launch_bounds__(512, 1) void qgemm_kernel(GemmArgs a) {
     if (lane == 0)
 #pragma unroll
         for (int u = 0; u < NX; ++u) k_s[wave * NX + u] = kx[u] == kNone ? 0 : kx[u];
+    if (tid == 0) lds.nan = 0;
     __syncthreads();
 #pragma unroll
     for (int i = tid; i < TM * TN; i += 512) {
@@ -617,6 +668,24 @@ __global__ __launch_bounds__(512, 1) void qgemm_kernel(GemmArgs a) {
 #pragma unroll
         for (int q = 1; q < KQ; ++q) v += y_s[q * TM * TN + i];
         a.y[(size_t)(t0 + tok) * a.rows + r0 + row] = __builtin_amdgcn_ldexpf(v, -k_s[tok]);
+        if (g_dense<TY>() && !INF && v != v) lds.nan = 1;
+    }
+}
+
+// The split gives NaN where an infinite x or a dense row's infinite weight
+// makes a product infinite (inf - inf in the residual, 0 times inf beside an
+// x that f16 holds).  The block formats' matvec does so too; the dense one
+// gives inf.  So a dense tile with a NaN among its results is done again with
+// both kept finite in one of the two products: the same sums elsewhere.
+// (Testing for them in the first pass cost 3 to 8% of every call.)  An x that
+// is 0 in f16 once scaled, 2^-36 of the token's largest, still counts as 0.
+template <int TY, int TT, int RT, int WR>
+__global__ __launch_bounds__(512, 1) void qgemm_kernel(GemmArgs a) {
+    __shared__ GemmLds<TY, TT, RT, WR> lds;
+    qgemm_tile<TY, TT, RT, WR, false>(a, lds);
+    if constexpr (g_dense<TY>()) {
+        __syncthreads();
+        if (__builtin_amdgcn_readfirstlane(lds.nan)) qgemm_tile<TY, TT, RT, WR, true>(a, lds);
     }
 }
 

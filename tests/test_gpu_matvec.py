@@ -252,3 +252,41 @@ def test_gemm_small_x_keeps_its_bits(name, n_tok):
         err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
         say(f"gemm {name} n_tok={n_tok} x rms {rms}: {err:.2e}")
         assert err <= 2.0 ** -21, (name, rms, err)
+
+
+@pytest.mark.parametrize("name", ["f16", "bf16"])
+@pytest.mark.parametrize("n_tok", [4, 20, 70])
+def test_dense_infinite_and_nan(name, n_tok):
+    # products and sums that are infinite or NaN come out as the fp32 matvec
+    # (4 tokens) has them, and touch no other token or row
+    rows, in_dim = 70, 512
+    w = oracle.quant_weights(oracle.QTYPES[name], rows, in_dim, 88).view(np.uint16).reshape(rows, in_dim).copy()
+    inf, nan = (0x7C00, 0x7E00) if name == "f16" else (0x7F80, 0x7FC0)
+    w[3, 100] = inf
+    w[4, 300] = inf | 0x8000
+    w[5, [7, 411]] = inf, inf | 0x8000  # inf - inf, where the x agree in sign
+    w[6, 90] = nan
+    w[8] &= 0x8000                      # 0 times an infinite x
+    if name == "bf16":
+        w[3, 102:108] = 0x7149          # 1e30 beside the infinite weight
+    x = oracle.normal(89, (n_tok, in_dim))
+    x[1, 200] = np.inf
+    x[2, [30, 31]] = np.inf, -np.inf
+    x[3, 511] = np.nan
+    if n_tok > 4:
+        x[9, 100] = -np.inf             # meets the infinite weight
+        x[10, 100] = 0.0                # and 0 does
+        x[11] *= np.float32(1e36)       # large beside infinite weights
+        x[12, :] = 0.0
+        x[12, 5] = np.inf               # before any nonzero x
+    w = w.reshape(-1).view(np.uint8)
+    got = gemm(name, w, rows, in_dim, x).astype(np.float64)
+    W = oracle.dequant(oracle.QTYPES[name], w, rows * in_dim).reshape(rows, in_dim).astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        ref = np.stack([(W * xt.astype(np.float64)).sum(-1) for xt in x])
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)])
+    for t in range(n_tok):
+        f = np.isfinite(ref[t])
+        if f.any():
+            assert np.abs(got[t, f] - ref[t, f]).max() <= 3e-5 * np.abs(ref[t, f]).max(), t
