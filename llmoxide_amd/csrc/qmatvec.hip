@@ -14,8 +14,8 @@
 // Work split (the direct kernel; the staged one is described at
 // qmatvec_lds_kernel).  A workgroup of four waves stages x [n_tok, in_dim] in LDS once,
 // then its waves take row groups of RW = 4 rows in turn (the grid is capped,
-// so a workgroup serves many groups).  Lane l takes 64-weight units l,
-// l + 64, ... of the rows (a Q6_K unit is a quarter of a half-block), reads
+// so a workgroup serves many groups).  Lane l takes units l, l + 64, ... of the
+// rows (64 weights; a Q6_K unit is a quarter of a half-block, a dense one 16 bytes), reads
 // the unit's x from LDS once per token for all RW rows, and streams the rows'
 // weight bytes from HBM once (no reuse).  Rows end with a DPP wave sum.
 // Quants reach float through v_cvt_f32_ubyte on bytewise-assembled dwords;
@@ -307,16 +307,36 @@ __device__ __forceinline__ void unit_dot(const uint8_t* const (&row)[RW], int uw
                 acc[r][t] += d0 * (s0 - 128.f * X0[t]) + d1 * (s1 - 128.f * X1[t]);
             }
         }
-    } else {
-        // dense rows: U consecutive weights, one 16-byte load a row, every
-        // row's issued before the first is used
-        constexpr int U = QTraits<TY>::unit;
-        typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-        const float* xc = xs + U * ux;
-        u32x4 v[RW];
+    }
+}
+
+// Dense rows: unit u is U = QTraits::unit consecutive weights, 16 bytes of each
+// row.  A lane's NU units are loaded before the first is used.  f16 and bf16
+// pin the loads there: the scheduler sank some between the products, and a
+// matrix of few rows, whose waves have little else in flight, then took longer
+// than with 64-weight units, which load 512 bytes a lane at once.  us a call,
+// 64-weight units / unpinned / pinned: f16, four tokens x 512 x 4096 11.0 /
+// 19.8 / 8.7; bf16, one token x 256 x 4096 6.5 / 9.9 / 5.7, x 64 x 16384 18.5 /
+// 24.2 / 10.4, x 12288 x 4096 73.5 / 18.4 / 16.0.  f32 streams a large matrix
+// faster unpinned, in fewer registers (one token x 12288 x 4096 35.1, pinned
+// 37.0), but for four tokens (x 256 x 4096 12.1 / 13.8 / 10.4).
+template <int TY, int T>
+constexpr int dense_units() { return T == 4 && TY != kBF16 ? 8 : TY == kF32 ? 1 : 4; }
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+template <int TY, int T, int RW, int NU>
+__device__ __forceinline__ void dense_dot(const uint8_t* const (&row)[RW], int u0, const float* xs, int in_dim,
+                                          float (&acc)[RW][T]) {
+    constexpr int U = QTraits<TY>::unit;
+    u32x4 v[NU][RW];
+#pragma unroll
+    for (int n = 0; n < NU; ++n)
 #pragma unroll
         for (int r = 0; r < RW; ++r)
-            v[r] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(row[r] + (size_t)16 * uw));
+            v[n][r] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(row[r] + (size_t)16 * (u0 + 64 * n)));
+    if constexpr (NU > 1) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int n = 0; n < NU; ++n) {
+        const float* xc = xs + U * (u0 + 64 * n);
 #pragma unroll
         for (int t = 0; t < T; ++t) {
             float xv[U];
@@ -331,7 +351,7 @@ __device__ __forceinline__ void unit_dot(const uint8_t* const (&row)[RW], int uw
                 float s = 0.f;
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    const uint32_t wv = v[r][j];
+                    const uint32_t wv = v[n][r][j];
                     if constexpr (TY == kF32) {
                         s = fmaf(__builtin_bit_cast(float, wv), xv[j], s);
                     } else if constexpr (TY == kF16) {
@@ -391,9 +411,19 @@ __global__ __launch_bounds__(kQmvWaves * 64) void qmatvec_kernel(QmvArgs a) {
         for (int r = 0; r < kQmvRows; ++r)
 #pragma unroll
             for (int t = 0; t < T; ++t) acc[r][t] = 0.f;
-        constexpr int UNROLL = QTraits<TY>::unit < 64 ? 4 : 1;  // dense units are one load a row
-#pragma unroll UNROLL
-        for (int u = lane; u < n_units; u += 64) unit_dot<TY, T, false, kQmvRows>(row, u, u, xs, a.in_dim, acc);
+        if constexpr (QTraits<TY>::unit < 64) {
+            constexpr int NU = dense_units<TY, T>();
+            int u = lane;
+            if constexpr (NU > 4)
+                for (; u - lane + 64 * NU <= n_units; u += 64 * NU)
+                    dense_dot<TY, T, kQmvRows, NU>(row, u, xs, a.in_dim, acc);
+            if constexpr (NU > 1)
+                for (; u - lane + 64 * 4 <= n_units; u += 64 * 4) dense_dot<TY, T, kQmvRows, 4>(row, u, xs, a.in_dim, acc);
+#pragma unroll 4
+            for (; u < n_units; u += 64) dense_dot<TY, T, kQmvRows, 1>(row, u, xs, a.in_dim, acc);
+        } else {
+            for (int u = lane; u < n_units; u += 64) unit_dot<TY, T, false, kQmvRows>(row, u, u, xs, a.in_dim, acc);
+        }
 #pragma unroll
         for (int r = 0; r < kQmvRows; ++r) {
 #pragma unroll

@@ -71,6 +71,15 @@ def test_partial_and_multiple_chunks(name, rows, in_dim, n_tok):
     run(name, rows, in_dim, n_tok, seed=11 + rows + n_tok)
 
 
+@pytest.mark.parametrize("name,in_dim", [("f32", 2048), ("f32", 3648), ("f16", 2048), ("f16", 4096), ("f16", 3776),
+                                         ("bf16", 2048), ("bf16", 3776)])
+@pytest.mark.parametrize("n_tok", [1, 2, 3, 4])
+def test_dense_unit_loops(name, in_dim, n_tok):
+    # rows of whole 8-unit and 4-unit steps a lane, and of each with single
+    # units and a last one that only some lanes have
+    run(name, 21, in_dim, n_tok, seed=100 + in_dim + n_tok)
+
+
 # ---- the matrix-core GEMM (n_tok >= 16, Q4_K / Q6_K / Q8_0): same bar --
 GEMM_TYPES = ["q4_k", "q6_k", "q8_0"]
 
