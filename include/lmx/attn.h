@@ -369,7 +369,7 @@ lmx_status lmx_deltanet_back(const lmx_delta_back_desc *d, float *o, const float
  *   x  [n_tok, in_dim] f32, y [n_tok, rows] f32, 16-byte aligned, disjoint
  * in_dim: a multiple of 256 (Q4_K, Q6_K) or 64 (the others), at most 16384.
  * A few tokens (and every batch of F32 weights) go four per launch, each
- * launch reading W once.  From 5 to 16 tokens on, by type and rows (the
+ * launch reading W once.  From 5 to 16 tokens on, by type and shape (the
  * reference's GEMM_MIN_TOKENS is 16, crates/gpu/src/lib.rs:1083; its GEMM is
  * gemm_q6k, gemm.wgsl:93-95), the other types go through one matrix-core GEMM
  * launch that reads W once (block formats: in_dim a multiple of 128); it

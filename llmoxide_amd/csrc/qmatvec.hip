@@ -571,27 +571,40 @@ static lmx_status launch_type(const QmvArgs& a, int T, hipStream_t st) {
 lmx_status qgemm(const lmx_qmv_desc* d, const void* w, const float* x, float* y, hipStream_t st);
 
 // Tokens from which the GEMM is the faster one.  It reads W once and takes about
-// the same time up to 32 tokens, the matvec a launch per four.  At in_dim 4096,
-// us at 4 / 8 / 12 tokens against the GEMM: Q6_K 1024 rows 8 / 16 / 24 : 28,
-// 4096 rows 17 / 33 / 49 : 29; Q8_0 4096 rows 26 / 50 / 74 : 23; bf16 4096
-// rows 13 / 26 / 38 : 26.  So: with the third launch, with the second where rows or
-// bytes are many, with the fourth for a short Q6_K matrix.  Q4_K waits for the
-// reference's 16: the GEMM's offset term, split into f16 parts, is 2.0e-7 from
-// the exact sums where the matvec is 1.6e-7 (the other types' GEMM is the
-// closer one).  fp32 weights stay with the matvec.
-static uint32_t gemm_min_tokens(uint32_t type, uint32_t rows) {
-    if (type == kF32) return UINT32_MAX;
-    if (type == kQ4K) return 16;
-    if (type == kF16 || type == kBF16) return 9;
-    if (type == kQ6K && rows < 2048) return 13;
-    return rows >= (type == kQ8_0 ? 2048u : 8192u) ? 5 : 9;
+// the same time up to 32 tokens, the matvec a launch per four, each a second
+// round of workgroups above 2048 rows.  us at 4 / 8 / 12 tokens against the GEMM:
+//   Q6_K  in_dim 4096: 2048 rows 8 / 17 / 24 : 28 (13 tokens 27), 2560 rows 16 /
+//         29 / 43 : 28, 8192 rows 29 / 58 / 86 : 29; in_dim 2048, 2048 rows, 9
+//         tokens 17 : 16; 13 tokens at in_dim 2304 22 : 17, 8192 57 : 52 (above
+//         4096 the matvec's LDS holds fewer tokens a launch)
+//   Q8_0  in_dim 4096: 2048 rows 13 / 24 / 37 : 23 (7 tokens 21), 2560 rows 24 /
+//         45 / 75 : 23; in_dim 2048, 5 tokens 12.1 : 12.7, 6 14 : 13; in_dim
+//         8192, 7 tokens 43 : 41
+//   bf16  in_dim 4096: 4096 rows 10 / 20 / 30 : 26, 64 rows 8 / 16 / 24 : 24
+// (Q6_K and Q8_0 of a few rows: the matvec has one or two of its two-row groups
+// a workgroup and none waits for another; Q8_0 4 rows x 4096, 10 tokens 20 : 22.)
+// Q4_K waits for the reference's 16: the GEMM's offset term, split into f16
+// parts, is 1.8e-7 from the exact sums where the matvec is 1.6e-7 (Q6_K's and
+// Q8_0's GEMM is the closer one).  fp32 weights stay with the matvec.
+static uint32_t gemm_min_tokens(uint32_t type, uint32_t rows, uint32_t in_dim) {
+    switch (type) {
+        case kF32: return UINT32_MAX;
+        case kQ4K: return 16;
+        case kQ6K:
+            if (rows < 8) return in_dim <= 2048 ? 13 : 16;
+            return rows >= 8192 ? 5 : rows > 2048 || in_dim <= 2048 ? 9 : in_dim > 3072 && in_dim <= 4096 ? 14 : 13;
+        case kQ8_0:
+            if (rows < 8) return in_dim <= 2048 ? 9 : 16;
+            return rows > 2048 ? 5 : in_dim <= 2048 ? 6 : in_dim <= 4096 ? 8 : 7;
+        default: return 9;  // f16, bf16
+    }
 }
 
 // Host side: tokens go in tiles of up to kQmvMaxTok (each tile re-reads W),
 // or to the GEMM.
 lmx_status qmatvec(const lmx_qmv_desc* d, const void* w, const float* x, float* y, hipStream_t st) {
     const bool dense = d->type == kF32 || d->type == kF16 || d->type == kBF16;
-    if (d->n_tok >= gemm_min_tokens(d->type, d->rows) && (dense || d->in_dim % 128 == 0))
+    if (d->n_tok >= gemm_min_tokens(d->type, d->rows, d->in_dim) && (dense || d->in_dim % 128 == 0))
         return qgemm(d, w, x, y, st);
     int unit = 0;  // of the shape check
     size_t bb = 0, be = 0;

@@ -131,11 +131,18 @@ def test_gemm_one_and_three_chunks(in_dim):
     run("q8_0", 130, in_dim, 70, seed=70 + in_dim)
 
 
-@pytest.mark.parametrize("name", GEMM_TYPES)
-def test_matvec_and_gemm_agree_across_the_threshold(name):
-    # 15 tokens take the matvec tiles, 16 the GEMM: both match the oracle
-    for n_tok in (15, 16):
-        run(name, 256, 1024, n_tok, seed=60)
+# (type, rows, in_dim, tokens from which the GEMM runs: gemm_min_tokens)
+THRESHOLDS = [("q4_k", 256, 1024, 16), ("q6_k", 7, 2304, 16), ("q6_k", 256, 1024, 9), ("q6_k", 256, 2304, 13), ("q6_k", 40, 4096, 14),
+              ("q6_k", 2049, 2304, 9), ("q6_k", 8192, 768, 5), ("q8_0", 7, 1024, 9), ("q8_0", 7, 2304, 16),
+              ("q8_0", 256, 1024, 6), ("q8_0", 256, 2304, 8), ("q8_0", 256, 4224, 7), ("q8_0", 2049, 384, 5),
+              ("f16", 256, 1024, 9), ("bf16", 256, 1024, 9)]
+
+
+@pytest.mark.parametrize("name,rows,in_dim,n_min", THRESHOLDS)
+def test_matvec_and_gemm_agree_across_the_threshold(name, rows, in_dim, n_min):
+    # the last batch that takes the matvec and the first that takes the GEMM
+    for n_tok in (n_min - 1, n_min):
+        run(name, rows, in_dim, n_tok, seed=60)
 
 
 @pytest.mark.parametrize("name", GEMM_TYPES)
