@@ -184,7 +184,8 @@ lmx_status lmx_attn_prologue(const lmx_prologue_desc *d, float *q, const float *
  * lmx_workspace_init; 0 bytes may be asked for (ws may then be NULL).  It
  * holds the split partials of decode, and of prefill when a short batch on a
  * long cache, or a causal batch of fp32 queries, is cut into key splits to
- * fill the GPU.
+ * fill the GPU (for a long batch of fp32 queries at head_dim 128, at most 80
+ * MiB, and the call runs on another kernel in less).
  * head_dim: the kernels run 64, 128, 256 and 512 natively (rows 16-byte
  * aligned: kv_dim and q_stride multiples of 8, buffers 16-byte aligned).  Any
  * other multiple of 4 up to 512 (the reference's vec4 domain, attn.wgsl:36-46;
@@ -211,10 +212,10 @@ lmx_status lmx_attn_fwd(const lmx_attn_params *p, const void *q, lmx_dtype q_dt,
  * lmx_attn_fwd; the split partials go to a library-owned scratch array of
  * LMX_NOALLOC_SCRATCH_BYTES per GPU (resident from the library's first use
  * on that GPU until the process ends).  Returns LMX_E_WORKSPACE, enqueuing
- * nothing, when the call cannot do with that.  (A long prefill with fp32
- * queries that lmx_attn_workspace_bytes offers more than this for, and that
- * can do with less, runs with fewer key splits: the same to rounding.)  A
- * 32k-token decode at Qwen3-8B shape needs about 2 MiB, a
+ * nothing, when the call cannot do with that.  (Where
+ * lmx_attn_workspace_bytes offers a long prefill with fp32 queries more than
+ * this, the call runs on the kernel that does with less: the same to
+ * rounding.)  A 32k-token decode at Qwen3-8B shape needs about 2 MiB, a
  * 512-token chunk on a 4k cache about 34 MiB.  No entry point allocates,
  * and this one takes no workspace either.  The scratch used is that of the
  * device `stream` belongs to (the current device for the null stream).

@@ -1370,6 +1370,14 @@ int prefill_wide_rows(int hd);
 int prefill_wide_gp(int G);
 lmx_status prefill_wide(const PrefillArgs& a, int hd, lmx_dtype q_dt, bool lin, hipStream_t st);
 
+static size_t round_up256(size_t x) { return (x + 255) / 256 * 256; }
+
+static size_t split_bytes(const lmx_attn_params* p, int sp) {
+    if (sp == 1) return 0;
+    const size_t rows = (size_t)sp * p->n_tokens * p->n_heads;
+    return round_up256(rows * 2 * sizeof(float)) + round_up256(rows * p->head_dim * sizeof(float));
+}
+
 // Estimated time of a head_dim 128 call with fp32 queries in us: workgroups of
 // bm rows, their key ranges cut into sp splits, tile_us per 64-key tile, one
 // workgroup a CU, heaviest first.  The longest unit bounds it from below, and
@@ -1398,7 +1406,16 @@ static float f32_prefill_us(const lmx_attn_params* p, int bm, int sp, float tile
 // heads); the kernel they choose is the faster one or within 5% of it.  At
 // 32 heads on 8, 128-row kernel : ping-pong, us a call: 512 tokens 25 : 32,
 // 2048 81 : 87, 3000 171 : 130, 4000 273 : 204; 512 tokens at position 4096
-// 83 : 73, 2048 there 314 : 264.
+// 83 : 73, 2048 there 314 : 264.  At positions up to 60000 and 8 to 64 heads
+// the choice stays within 5% of the faster kernel.
+// The splits' partials are held to 80 MiB, little more than the 128-row kernel
+// takes at most: the estimate alone asked for up to 435 MiB (64 heads, 6528
+// tokens at position 30000), which a caller without a workspace of its own
+// allocates and clears for each call.  Fewer splits, or none, cost some of the
+// gain at long positions (16 heads, 4608 tokens at 30000, 128-row kernel / held
+// / unbounded: 2885 / 1972 / 1748; 40 heads, 2048 at 4096 477 / 391 / 376; 32
+// heads, 1500 at 4096 261 / 213 / 224).
+constexpr size_t kMaxSplitBytes = (size_t)80 << 20;
 static int ping_pong_f32_splits(const lmx_attn_params* p, int tile_splits) {
     const int forced = tuning().prefill_kernel;
     if (p->head_dim != 128 || forced == 0) return 0;
@@ -1406,6 +1423,7 @@ static int ping_pong_f32_splits(const lmx_attn_params* p, int tile_splits) {
     float best_us = forced == 1 ? 3.4e38f : f32_prefill_us(p, kPfBM, tile_splits, 2.3f);
     const long longest = ((long)p->base_pos + p->n_tokens) / 64;
     for (int sp = 1; sp <= kMaxSplits && (sp == 1 || longest >= 4 * sp); ++sp) {
+        if (sp > 1 && split_bytes(p, sp) > kMaxSplitBytes) break;
         const float us = 4.f + f32_prefill_us(p, kPpBM, sp, 2.7f);
         if (us < best_us) {
             best = sp;
@@ -1433,14 +1451,6 @@ static int prefill_splits(const lmx_attn_params* p, lmx_dtype q_dt) {
     if (sp > tiles / min_tiles) sp = tiles / min_tiles;
     if (sp > max_splits) sp = max_splits;
     return sp < 2 ? 1 : (int)sp;
-}
-
-static size_t round_up256(size_t x) { return (x + 255) / 256 * 256; }
-
-static size_t split_bytes(const lmx_attn_params* p, int sp) {
-    if (sp == 1) return 0;
-    const size_t rows = (size_t)sp * p->n_tokens * p->n_heads;
-    return round_up256(rows * 2 * sizeof(float)) + round_up256(rows * p->head_dim * sizeof(float));
 }
 
 // The workspace without which a call is refused: the 128-row kernel's (f16

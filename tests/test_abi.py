@@ -317,6 +317,21 @@ def test_decode_workspace_grows_with_the_context():
             prev = b
 
 
+def test_prefill_workspace_is_bounded():
+    """The key splits offered to a prefill call never ask for more than 80 MiB,
+    however long the cache and however many heads: a caller without a
+    workspace of its own allocates and clears it for each call."""
+    L = lmx.lib()
+    for H, Hkv in ((8, 8), (16, 8), (32, 8), (40, 8), (64, 8), (71, 1)):
+        for hd in (64, 128, 256, 512):
+            for t in (9, 100, 512, 896, 1920, 2816, 4096, 4608, 5000, 6528, 16384):
+                for base in (0, 700, 4096, 30000, 120000):
+                    for bidi in (False, True):
+                        p = _params(n_tokens=t, n_heads=H, n_kv_heads=Hkv, head_dim=hd, base_pos=base,
+                                    n_slots=base + t, bidi=bidi)
+                        assert L.lmx_attn_workspace_bytes(ctypes.byref(p)) <= 80 << 20, (H, hd, t, base, bidi)
+
+
 def test_decode_workspace_covers_few_token_batches():
     L = lmx.lib()
     for base in (100, 5000, 32000):
