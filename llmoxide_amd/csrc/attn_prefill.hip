@@ -1364,11 +1364,9 @@ static int prefill_gp(int G) {
 constexpr int kMinSplitTiles = 8;
 constexpr int kMaxSplits = 16;
 constexpr int kCus = 256;
-int decode_max_vis(const lmx_attn_params* p);
 // attn_prefill_wide.hip: head_dim 256 and 512
-int prefill_wide_rows(int hd);
-int prefill_wide_gp(int G);
-lmx_status prefill_wide(const PrefillArgs& a, int hd, lmx_dtype q_dt, bool lin, hipStream_t st);
+WidePlan prefill_wide_plan(const lmx_attn_params* p, lmx_dtype q_dt);
+lmx_status prefill_wide(const PrefillArgs& a, int hd, lmx_dtype q_dt, bool lin, bool few, hipStream_t st);
 
 static size_t round_up256(size_t x) { return (x + 255) / 256 * 256; }
 
@@ -1437,8 +1435,9 @@ static int prefill_splits(const lmx_attn_params* p, lmx_dtype q_dt) {
     const int hd = (int)p->head_dim;
     const bool wide = hd >= 256;
     const int G = (int)(p->n_heads / p->n_kv_heads);
-    const int gp = wide ? prefill_wide_gp(G) : prefill_gp(G);
-    const long bm = wide ? prefill_wide_rows(hd) / gp : kPfBM / gp;
+    const WidePlan wp = wide ? prefill_wide_plan(p, q_dt) : WidePlan{};
+    const int gp = wide ? wp.gp : prefill_gp(G);
+    const long bm = wide ? wp.tokens : kPfBM / gp;
     const long n_wg = (long)((p->n_tokens + bm - 1) / bm) * (p->n_heads / gp);
     const long slots = (long)kCus * (wide || (hd == 128 && q_dt != LMX_F16) ? 1 : 2);
     if (n_wg >= slots) return 1;
@@ -1512,8 +1511,9 @@ lmx_status prefill_fwd(const lmx_attn_params* p, const AttnIo& io, const void* q
     window_magic((uint32_t)a.window, &a.w_magic, &a.w_shift);
     const int hd = (int)p->head_dim;
     const bool wide = hd >= 256;
-    a.gp = wide ? prefill_wide_gp(a.G) : prefill_gp(a.G);
-    const int bm = wide ? prefill_wide_rows(hd) / a.gp : pp ? kPpBM / a.gp : kPfBM / a.gp;
+    const WidePlan wp = wide ? prefill_wide_plan(p, q_dt) : WidePlan{};
+    a.gp = wide ? wp.gp : prefill_gp(a.G);
+    const int bm = wide ? wp.tokens : pp ? kPpBM / a.gp : kPfBM / a.gp;
     a.n_qtiles = (a.n_tokens + bm - 1) / bm;
     long nblk = (long)a.n_qtiles * (a.H / a.gp) * a.n_split;
     // Linear addressing: no k_cur rows and every position below the window;
@@ -1548,7 +1548,7 @@ lmx_status prefill_fwd(const lmx_attn_params* p, const AttnIo& io, const void* q
         else hipLaunchKernelGGL((attn_prefill_pp_kernel<QT, 128, false>), grid, dim3(512), 0, st, a);   \
     } while (0)
     if (wide) {
-        const lmx_status s = prefill_wide(a, hd, q_dt, lin, st);
+        const lmx_status s = prefill_wide(a, hd, q_dt, lin, wp.few, st);
         if (s != LMX_OK) return s;
     } else if (kh) {  // f16 queries only
         if (hd == 64) hipLaunchKernelGGL((attn_prefill_kh_kernel<f16, 64>), grid, dim3(256), 0, st, a);

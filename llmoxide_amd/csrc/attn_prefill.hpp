@@ -30,6 +30,16 @@ struct PrefillArgs {
     float* part_ml;  // [n_split][t][H][2]
 };
 
+// How attn_prefill_wide_kernel runs a call: query heads and tokens of a
+// workgroup, and whether in its form for few rows.
+struct WidePlan {
+    int gp, tokens;
+    bool few;
+};
+
+// Keys the call's last query sees at most (attn_decode.hip).
+int decode_max_vis(const lmx_attn_params* p);
+
 constexpr float kRescaleSlack = 8.f;  // log2 units a running max may lag by
 
 // attn.wgsl:52-66

@@ -49,7 +49,15 @@
 namespace lmx {
 
 // LIN: key row p lives at cache row p (see attn_prefill_kernel).
-template <typename QT, int HD, bool LIN>
+// FEW: the workgroup's rows are at most few_rows(HD), one row block.  Q then
+// leaves the first tile's LDS free, whose transfers go out with Q's instead of
+// after it, and the other row blocks' waves only move data.  us a call of 9
+// tokens, head_dim 256, 16 heads on 8, position 0, the kernel this file
+// replaces / not FEW / FEW: fp32 queries 11.0 / 14.1 / 10.8, f16 8.5 / 10.6 /
+// 8.3; head_dim 512, f16 9.7 / 10.8 / 8.3.
+template <int HD>
+constexpr int few_rows() { return HD == 256 ? 32 : 16; }
+template <typename QT, int HD, bool LIN, bool FEW>
 __global__ __launch_bounds__(512, 1) void attn_prefill_wide_kernel(PrefillArgs a) {
     static_assert(HD == 256 || HD == 512, "two or four waves a row block");
     constexpr bool kQlo = sizeof(QT) == 4;  // fp32 queries carry an f16 residual (qk_tile)
@@ -110,7 +118,7 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_wide_kernel(PrefillArgs a
     const int kb = j4 & 1, dq = j4 >> 1;         // score block and dim part
     const int t = a.n_tokens, base = a.base_pos, w = a.window;
     const int end = base + t - 1;
-    const int tpw = scalar(BM / gp), tpb = scalar(32 / gp);  // tokens of the workgroup, of a row block
+    const int tpw = scalar((FEW ? few_rows<HD>() : BM) / gp), tpb = scalar(32 / gp);  // tokens of the workgroup, of a row block
     const int q0 = qt * tpw, qb0 = q0 + rb * tpb;
 
     // ---- this lane's row: token qb0 + l32 / gp, head l32 % gp of the group.
@@ -210,23 +218,38 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_wide_kernel(PrefillArgs a
     // back)
     const int gp_shift = __builtin_ctz(gp);
     constexpr int ROWQ = HD * (int)sizeof(QT);
+    const int nq = FEW ? scalar(min(tpw, t - q0) * gp) : BM;  // rows
     f16* Q_s = kQlo ? K_st(0) : V_st(0);
-    if (!kQlo && n_t > 0) fetch(a.k, a.k_cur, kt_begin, K_st(0), false);
+    if constexpr (FEW) {  // beside the first tile: the second stage of V, or X_s
+        static_assert(HD == 256 || !kQlo, "16 rows of f16 fill X_s");
+        Q_s = HD == 256 ? V_st(1) : reinterpret_cast<f16*>(X_s);
+        static_assert(few_rows<HD>() * ROWQ <= (HD == 256 ? TILE * 2 : (int)sizeof(X_s)), "Q's rows fit there");
+    } else if (!kQlo && n_t > 0) {
+        fetch(a.k, a.k_cur, kt_begin, K_st(0), false);
+    }
+    constexpr int NQ = BM * ROWQ / 1024 / 8;  // transfers a wave issues for BM rows
 #pragma unroll 4
-    for (int i = 0; i < BM * ROWQ / 1024 / 8; ++i) {
-        const int n = wave * (BM * ROWQ / 1024 / 8) + i;
+    for (int i = 0; i < (FEW ? (nq * ROWQ + 1023) / 1024 - wave : 8 * NQ); i += 8) {
+        const int n = FEW ? wave + i : wave * NQ + i / 8;
         const int at = n * 1024 + lane * 16, r = at / ROWQ, c = at % ROWQ / 16;
         const int qt_r = min(q0 + (r >> gp_shift), t - 1), h_r = kvh * a.G + hg * gp + (r & (gp - 1));
         dma16_lane(reinterpret_cast<const char*>(a.q) + ((size_t)qt_r * a.H + h_r) * a.q_stride * sizeof(QT) +
                        ((c ^ (r & 15)) << 4),
                    lds_addr(Q_s) + n * 1024);
     }
-    wait_dma<0>();
+    if (FEW && n_t > 0) {
+        fetch(a.k, a.k_cur, kt_begin, K_st(0), false);
+        fetch(a.v, a.v_cur, kt_begin, V_st(0), true);
+        wait_dma<2 * NDMA>();  // Q: the tile took that many transfers or more
+    } else {
+        wait_dma<0>();
+    }
     __syncthreads();
     f16x8 qf[KSTEPS], ql[kQlo ? KSTEPS : 1];
     float c_sc = a.c;
     {
-        const int r = rb * 32 + l32;
+        // (FEW: rows past the batch, and the idle waves', read its last token's)
+        const int r = FEW && rb * 32 + l32 >= nq ? nq - gp + l32 % gp : rb * 32 + l32;
         const char* qrow_s = reinterpret_cast<const char*>(Q_s) + r * ROWQ;
         auto chunk = [&](int c) { return qrow_s + ((c ^ (r & 15)) << 4); };
         if constexpr (!kQlo) {
@@ -265,12 +288,13 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_wide_kernel(PrefillArgs a
         }
         settle_q(qf);
     }
-    __syncthreads();  // Q is in registers: its LDS is the tiles'
-    if (n_t > 0) {
+    if constexpr (!FEW) __syncthreads();  // Q is in registers: its LDS is the tiles'
+    if (!FEW && n_t > 0) {
         if (kQlo) fetch(a.k, a.k_cur, kt_begin, K_st(0), false);
         fetch(a.v, a.v_cur, kt_begin, V_st(0), true);
     }
 
+    const bool act = !FEW || rb == 0;
     for (int it = 0; it < n_t; ++it) {
         const int kt = kt_begin + it * BN;
         const int stage = STG == 2 ? it & 1 : 0;
@@ -294,7 +318,7 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_wide_kernel(PrefillArgs a
 #pragma unroll
             for (int i = 0; i < 16; ++i) s[i] = 0.f;
             const f16* Ks = K_st(stage);
-            {
+            if (act) {
                 constexpr int D = kTight ? 3 : 4;  // operand reads ahead
                 int k_tile = k_at0;
                 opaque(k_tile);
@@ -320,7 +344,7 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_wide_kernel(PrefillArgs a
                 // each part finishes the 16 keys in its registers 0-7 and
                 // hands over registers 8-15, which the other finishes
 #pragma unroll
-                for (int g = 0; g < 2; ++g) {
+                for (int g = 0; g < 2 && act; ++g) {
                     f32x4 x;
 #pragma unroll
                     for (int i = 0; i < 4; ++i) x[i] = s[8 + 4 * g + i] * c_sc;
@@ -362,19 +386,22 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_wide_kernel(PrefillArgs a
                 *reinterpret_cast<f16x8*>(&P_s[((rb * 4 + 2 * kb + dq + st) * 64 + lane) * 8]) = pf[st];
             }
         };
-        make_p();
-        f16x2 pm = {pf[0][0], pf[0][1]};
+        bool ask = false;
+        if (act) {
+            make_p();
+            f16x2 pm = {pf[0][0], pf[0][1]};
 #pragma unroll
-        for (int st = 0; st < PS; ++st)
+            for (int st = 0; st < PS; ++st)
 #pragma unroll
-            for (int j = 0; j < 8; j += 2) pm = __builtin_elementwise_max(pm, f16x2{pf[st][j], pf[st][j + 1]});
-        const float pmax = fmaxf((float)pm[0], (float)pm[1]);
-        bool ask = !(pmax <= kSlackP);
-        if (__builtin_amdgcn_ballot_w64(m_run < -1e29f) != 0) {  // a row's first keys set its max
-            float mt = sv[0];
+                for (int j = 0; j < 8; j += 2) pm = __builtin_elementwise_max(pm, f16x2{pf[st][j], pf[st][j + 1]});
+            const float pmax = fmaxf((float)pm[0], (float)pm[1]);
+            ask = !(pmax <= kSlackP);
+            if (__builtin_amdgcn_ballot_w64(m_run < -1e29f) != 0) {  // a row's first keys set its max
+                float mt = sv[0];
 #pragma unroll
-            for (int i = 1; i < NS; ++i) mt = fmaxf(mt, sv[i]);
-            ask = ask || (m_run < -1e29f && mt > -INFINITY);
+                for (int i = 1; i < NS; ++i) mt = fmaxf(mt, sv[i]);
+                ask = ask || (m_run < -1e29f && mt > -INFINITY);
+            }
         }
         const int asks = __builtin_amdgcn_ballot_w64(ask) != 0;
         if (lane == 0) F_s[wave] = asks;
@@ -406,9 +433,10 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_wide_kernel(PrefillArgs a
             const float shift = (mn > -1e29f ? mn : 0.f) - mb;
 #pragma unroll
             for (int i = 0; i < NS; ++i) sv[i] -= shift;
-            make_p();
+            if (act) make_p();
             __syncthreads();
         }
+        if (!act) continue;
         const f16x2 one2 = {(f16)1.f, (f16)1.f};
 #pragma unroll
         for (int st = 0; st < PS; ++st)
@@ -460,7 +488,7 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_wide_kernel(PrefillArgs a
 #pragma unroll
     for (int i = 0; i < WPR; ++i) l_tot += M_s[rb * WPR + i][l32];
     const bool part = n_split > 1;
-    if (part && qvalid && hh == 0 && j4 == 0)
+    if (part && act && qvalid && hh == 0 && j4 == 0)
         *reinterpret_cast<f32x2*>(a.part_ml + 2 * (((size_t)sp * t + qrow) * a.H + h)) = f32x2{m_run, l_tot};
     const float inv = part ? 1.f : 1.f / l_tot;
     char* O_s = reinterpret_cast<char*>(KV_s);
@@ -479,9 +507,10 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_wide_kernel(PrefillArgs a
     }
     __syncthreads();
     float* dst = part ? a.part_o + (size_t)sp * t * a.H * HD : a.out;
+    constexpr int NO = BM * ROWO / 1024 / 8;
 #pragma unroll 4
-    for (int i = 0; i < BM * ROWO / 1024 / 8; ++i) {
-        const int at = (wave * (BM * ROWO / 1024 / 8) + i) * 1024 + lane * 16;
+    for (int i = 0; i < (FEW ? nq * ROWO / 1024 - wave : 8 * NO); i += 8) {
+        const int at = (FEW ? wave + i : wave * NO + i / 8) * 1024 + lane * 16;
         const int r = at / ROWO, c = at % ROWO / 16;
         const int row_t = q0 + (r >> gp_shift), row_h = kvh * a.G + hg * gp + (r & (gp - 1));
         f32x4 y = *reinterpret_cast<const f32x4*>(O_s + r * ROWO + ((c ^ (r & 15)) << 4));
@@ -492,18 +521,32 @@ __global__ __launch_bounds__(512, 1) void attn_prefill_wide_kernel(PrefillArgs a
     }
 }
 
-// Query rows of a workgroup, and the heads that share them: the largest power
-// of two that divides the kv group, up to the 32 rows of a block.
-int prefill_wide_rows(int hd) { return hd == 512 ? 64 : 128; }
-int prefill_wide_gp(int G) {
-    if (const int v = tuning().prefill_gp; v > 0 && G % v == 0) return v;
-    int gp = 1;
+// Heads that share a workgroup's rows, its tokens, and which form it takes.
+// The heads: the largest power of two that divides the kv group, up to the 32
+// rows of a block.  A short call over few keys takes the FEW form with as few
+// heads as make one workgroup of its tokens, as long as the CUs hold all
+// workgroups at once.  The lines (us a call, not FEW / FEW): 64 heads on 8,
+// head_dim 256, f16, 32 tokens at position 900 25.4 / 21.5, at 16000 62 / 101;
+// 128 heads, 80 tokens at 900 38 / 58; head_dim 512, f16, 48 heads on 3, 17
+// tokens at 300 21.4 / 17.1, at 900 25.6 / 27.3; 64 heads on 8, 48 tokens at 900
+// 32 / 37.
+WidePlan prefill_wide_plan(const lmx_attn_params* p, lmx_dtype q_dt) {
+    const int hd = (int)p->head_dim, t = (int)p->n_tokens, H = (int)p->n_heads, G = H / (int)p->n_kv_heads;
+    const int few = hd == 256 ? few_rows<256>() : q_dt == LMX_F16 ? few_rows<512>() : 0;
+    const int most = hd == 512 ? 32 : q_dt == LMX_F16 ? 96 : 64, keys = hd == 512 ? 512 : 1024;
+    bool small = few && t <= most && decode_max_vis(p) <= keys;
+    int few_gp = 1, gp = 1;
+    while (2 * few_gp * t <= few && G % (2 * few_gp) == 0) few_gp *= 2;
     while (gp < 32 && G % (2 * gp) == 0) gp *= 2;
-    return gp;
+    small = small && (t * few_gp + few - 1) / few * (H / few_gp) < 256;
+    if (small) gp = few_gp;
+    if (const int v = tuning().prefill_gp; v > 0 && G % v == 0) gp = v;
+    if (few && (gp * t <= few || (small && gp <= few))) return {gp, few / gp, true};
+    return {gp, (hd == 512 ? 64 : 128) / gp, false};
 }
 
 // a: as prefill_fwd fills it, with gp, n_qtiles and n_split for this kernel.
-lmx_status prefill_wide(const PrefillArgs& a, int hd, lmx_dtype q_dt, bool lin, hipStream_t st) {
+lmx_status prefill_wide(const PrefillArgs& a, int hd, lmx_dtype q_dt, bool lin, bool few, hipStream_t st) {
     const long per_kvh = (long)a.n_qtiles * (a.G / a.gp) * a.n_split;
     long nblk = per_kvh * a.Hkv;
     if (a.Hkv % 8 && 8 % a.Hkv == 0) {
@@ -512,19 +555,25 @@ lmx_status prefill_wide(const PrefillArgs& a, int hd, lmx_dtype q_dt, bool lin, 
     }
     if (nblk > INT_MAX) return LMX_E_SHAPE;
     const dim3 grid((unsigned)nblk);
-#define LMX_WD(QT, HDV)                                                                                     \
-    do {                                                                                                    \
-        if (lin) hipLaunchKernelGGL((attn_prefill_wide_kernel<QT, HDV, true>), grid, dim3(512), 0, st, a);  \
-        else hipLaunchKernelGGL((attn_prefill_wide_kernel<QT, HDV, false>), grid, dim3(512), 0, st, a);     \
+#define LMX_WDL(QT, HDV, FEW)                                                                                   \
+    do {                                                                                                        \
+        if (lin) hipLaunchKernelGGL((attn_prefill_wide_kernel<QT, HDV, true, FEW>), grid, dim3(512), 0, st, a); \
+        else hipLaunchKernelGGL((attn_prefill_wide_kernel<QT, HDV, false, FEW>), grid, dim3(512), 0, st, a);    \
+    } while (0)
+#define LMX_WD(QT, HDV)                    \
+    do {                                   \
+        if (few) LMX_WDL(QT, HDV, true);   \
+        else LMX_WDL(QT, HDV, false);      \
     } while (0)
     if (q_dt == LMX_F16) {
         if (hd == 256) LMX_WD(f16, 256);
         else LMX_WD(f16, 512);
     } else {
         if (hd == 256) LMX_WD(float, 256);
-        else LMX_WD(float, 512);
+        else LMX_WDL(float, 512, false);
     }
 #undef LMX_WD
+#undef LMX_WDL
     return LMX_OK;
 }
 

@@ -92,3 +92,33 @@ def test_scores_that_grow_along_the_keys(hd):
     c.k16 = (c.kf * grow).astype(np.float16).view(np.uint16)
     c.kf = c.k16.view(np.float16).astype(np.float32)
     check(c, base=300, scale=1.0)
+
+
+@pytest.mark.parametrize("q_f16", [False, True])
+@pytest.mark.parametrize("t,H,Hkv,hd", [
+    (15, 4, 2, 256), (16, 4, 2, 256), (17, 4, 2, 256),       # two heads of 16 tokens fill 32 rows; one of 17
+    (9, 6, 2, 256), (32, 3, 3, 256), (33, 3, 3, 256), (64, 2, 1, 256), (65, 2, 1, 256),  # and two workgroups of tokens
+    (96, 2, 1, 256), (97, 2, 1, 256),
+    (9, 4, 1, 512), (16, 2, 1, 512), (17, 2, 1, 512), (32, 3, 3, 512), (33, 3, 3, 512)])
+def test_few_rows(t, H, Hkv, hd, q_f16):
+    # the form for few rows at its edges, from position 0, inside the second
+    # tile and over several
+    for base in (0, 50, 333):
+        check(AttnCase(t + base + hd, t=t, H=H, Hkv=Hkv, hd=hd, n_pos=base + t, q_f16=q_f16), base=base)
+
+
+@pytest.mark.parametrize("q_f16", [False, True])
+@pytest.mark.parametrize("hd", [256, 512])
+def test_few_rows_options(hd, q_f16):
+    # a ring with the batch beside it, every query seeing the whole batch, the
+    # output gate, and key splits (10 tokens of a head over 3000 keys)
+    c = AttnCase(hd + 7, t=20, H=4, Hkv=2, hd=hd, n_pos=220, q_f16=q_f16)
+    check(c, base=200, window=90)
+    gate = np.random.default_rng(6).standard_normal((c.t, c.H * hd)).astype(np.float32)
+    check(c, base=200, bidi=True, gate=gate)
+    check(AttnCase(hd + 8, t=10, H=2, Hkv=2, hd=hd, n_pos=3000, q_f16=q_f16), base=2990)
+    # scores that grow along the keys: every tile rescales
+    c = AttnCase(hd + 9, t=12, H=2, Hkv=2, hd=hd, n_pos=340, q_f16=q_f16)
+    c.k16 = (c.kf * np.linspace(0.05, 3.0, 340)[:, None]).astype(np.float16).view(np.uint16)
+    c.kf = c.k16.view(np.float16).astype(np.float32)
+    check(c, base=328, scale=1.0)
