@@ -1379,9 +1379,12 @@ static size_t split_bytes(const lmx_attn_params* p, int sp) {
 // Estimated time of a head_dim 128 call with fp32 queries in us: workgroups of
 // bm rows, their key ranges cut into sp splits, tile_us per 64-key tile, one
 // workgroup a CU, heaviest first.  The longest unit bounds it from below, and
-// so does the CUs' mean load plus what the last round leaves idle of the
-// lightest unit.  A split costs its partials' trip through memory (written
-// and read back at 3 TB/s) and the merge launch, 8 us.
+// so does the mean load of the busiest XCD plus what its last round leaves idle
+// of its lightest unit: with fewer than eight kv heads an XCD has only part of
+// one head's units, and the first of them the heaviest (taken for the mean of
+// all, 12 heads on 2, 1500 tokens were left on the 128-row kernel: 64, now 46).
+// A split costs its partials' trip through memory (written and read back at 3
+// TB/s) and the merge launch, 8 us.
 static float f32_prefill_us(const lmx_attn_params* p, int bm, int sp, float tile_us) {
     const int bn = 64;
     const long t = p->n_tokens, end = (long)p->base_pos + t, w = p->window;
@@ -1389,8 +1392,9 @@ static float f32_prefill_us(const lmx_attn_params* p, int bm, int sp, float tile
     const long units = (t + bm - 1) / bm * (long)p->n_heads * sp, rounds = (units + kCus - 1) / kCus;
     const long longest = (std::min(end, most + bm) + bn - 1) / bn;
     const long first = p->bidi ? longest : std::min<long>(longest, ((long)p->base_pos + bm + bn - 1) / bn);
-    const float load = 0.5f * (float)(first + longest) * (float)units / (float)sp / kCus +
-                       (float)(rounds * kCus - units) / kCus * (float)first / (float)sp;
+    const float light = (float)longest - (float)(longest - first) * std::min(1.f, (float)p->n_kv_heads / 8.f);
+    const float load = 0.5f * (light + (float)longest) * (float)units / (float)sp / kCus +
+                       (float)(rounds * kCus - units) / kCus * light / (float)sp;
     const float tiles = std::max((float)((longest + sp - 1) / sp), load);
     return tiles * tile_us + (sp > 1 ? 8.f + (float)t * (float)p->n_heads * 128.f * 8.f * (float)sp / 3e6f : 0.f);
 }
