@@ -288,11 +288,12 @@ def _stream(stream) -> Optional[int]:
     if stream is not None:
         return stream.cuda_stream
     torch = _torch()
-    if not torch.cuda.is_initialized():
+    # the raw handle alone, where this torch has it: a call of a few microseconds
+    # notices the torch.cuda.Stream object that current_stream() makes for it
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None:
         return torch.cuda.current_stream().cuda_stream
-    # the raw handle alone: a call of a few microseconds notices the
-    # torch.cuda.Stream object that current_stream() makes for it
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    return raw(torch.cuda.current_device())
 
 
 def _dt(t) -> int:

@@ -401,3 +401,16 @@ def test_padded_head_dims_validate_and_size_their_copies():
     pb = _params(head_dim=72)
     assert L.lmx_attn_decode_batched(ctypes.byref(pb), 1, 16, FAKE, FAKE, FAKE, FAKE, lmx.F32,
                                      lmx.F16, FAKE + (1 << 24), None, 0, None) == lmx.Status.E_UNSUPPORTED
+
+
+def test_current_stream_without_the_raw_handle(monkeypatch):
+    """torch builds without the private raw-handle call are asked for the
+    stream object; the handle is the current device's otherwise."""
+    from types import SimpleNamespace
+    cuda = SimpleNamespace(current_stream=lambda: SimpleNamespace(cuda_stream=77), current_device=lambda: 3)
+    monkeypatch.setattr(lmx, "_torch", lambda: SimpleNamespace(_C=SimpleNamespace(), cuda=cuda))
+    assert lmx._stream(None) == 77
+    raw = SimpleNamespace(_cuda_getCurrentRawStream=lambda dev: 100 + dev)
+    monkeypatch.setattr(lmx, "_torch", lambda: SimpleNamespace(_C=raw, cuda=cuda))
+    assert lmx._stream(None) == 103
+    assert lmx._stream(SimpleNamespace(cuda_stream=5)) == 5
