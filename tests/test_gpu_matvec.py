@@ -80,7 +80,7 @@ def test_dense_unit_loops(name, in_dim, n_tok):
     run(name, 21, in_dim, n_tok, seed=100 + in_dim + n_tok)
 
 
-# ---- the matrix-core GEMM (n_tok >= 16, Q4_K / Q6_K / Q8_0): same bar --
+# ---- the matrix-core GEMM (gemm_min_tokens): same bar --
 GEMM_TYPES = ["q4_k", "q6_k", "q8_0"]
 
 
@@ -120,14 +120,14 @@ def test_gemm_prefill_chunk_512(name):
 @pytest.mark.parametrize("name,in_dim", [("q4_k", 512), ("q6_k", 768), ("q8_0", 640)])
 @pytest.mark.parametrize("rows,n_tok", [(200, 33), (37, 16), (130, 65)])
 def test_gemm_ragged_edges(name, in_dim, rows, n_tok):
-    # rows and tokens off the 128 x 64 workgroup tile; Q6_K with 3 blocks a
-    # row puts odd rows 2 bytes off a dword; Q8_0 with 20 blocks a row
+    # rows and tokens off the tiles; Q6_K with 3 blocks a row puts odd rows 2
+    # bytes off a dword; Q8_0 with 20 blocks a row
     run(name, rows, in_dim, n_tok, seed=40 + rows + n_tok)
 
 
 @pytest.mark.parametrize("in_dim", [128, 384])
 def test_gemm_one_and_three_chunks(in_dim):
-    # the K loop runs two 128-weight chunks a round: one chunk, and an odd count
+    # rows of half a 256-weight chunk, and of one and a half
     run("q8_0", 130, in_dim, 70, seed=70 + in_dim)
 
 
@@ -192,8 +192,8 @@ def test_gemm_dense_edges(name, in_dim, rows, n_tok):
 @pytest.mark.parametrize("name,in_dim", [("q4_k", 768), ("q6_k", 256), ("q6_k", 1280), ("q8_0", 384)])
 @pytest.mark.parametrize("rows,n_tok", [(1, 16), (33, 32), (65, 64), (8200, 40), (16500, 17)])
 def test_gemm_row_tiles(name, in_dim, rows, n_tok):
-    # each tile of the dispatch: 32 and 64 rows beside 32 and 64 tokens, 64 x 128
-    # for the largest grids; the last row's bytes end the matrix
+    # 32-row tiles beside 32 and 64 tokens, and 64-row ones beside 32 (16500);
+    # the last row's bytes end the matrix
     run(name, rows, in_dim, n_tok, seed=120 + rows % 97 + n_tok)
 
 
@@ -306,3 +306,51 @@ def test_dense_infinite_and_nan(name, n_tok):
         f = np.isfinite(ref[t])
         if f.any():
             assert np.abs(got[t, f] - ref[t, f]).max() <= 3e-5 * np.abs(ref[t, f]).max(), t
+
+
+# ---- grids of a workgroup for every CU: 64 tokens x 64 rows, 64 x 128 (the
+# kernel of its own, qgemm_big.hip), and dense 32 tokens x 64 rows.  All rows
+# are computed; the first, some in the middle and the last are checked.
+def some_rows(rows):
+    return sorted(set(list(range(140)) + list(range(rows // 2, rows // 2 + 70)) + list(range(rows - 140, rows))))
+
+
+def run_some(name, rows, in_dim, n_tok, seed, x=None):
+    say(f"gemm {name} rows={rows} in_dim={in_dim} n_tok={n_tok}")
+    w = oracle.quant_weights(oracle.QTYPES[name], rows, in_dim, seed)
+    x = oracle.normal(seed + 50, (n_tok, in_dim)) if x is None else x
+    got, pick = gemm(name, w, rows, in_dim, x), some_rows(rows)
+    assert np.all(np.isfinite(got))
+    sub = np.ascontiguousarray(w.reshape(rows, -1)[pick]).reshape(-1)
+    ref = f64_ref(name, sub, len(pick), in_dim, x)
+    for t in range(n_tok):
+        err, scale = np.abs(got[t, pick] - ref[t]).max(), np.abs(ref[t]).max()
+        assert err <= 3e-5 * scale, f"{name} token {t}: max err {err} vs max |ref| {scale}"
+
+
+@pytest.mark.parametrize("name,in_dim", [("q4_k", 256), ("q4_k", 768), ("q6_k", 256), ("q6_k", 768), ("q8_0", 128),
+                                         ("q8_0", 384)])
+@pytest.mark.parametrize("rows,n_tok", [
+    (16400, 40), (16321, 64),                            # 64 x 64
+    (4090, 500), (32641, 33), (32768, 64), (8065, 257)])  # 64 x 128, whole and ragged
+def test_gemm_full_grids(name, in_dim, rows, n_tok):
+    run_some(name, rows, in_dim, n_tok, seed=140 + rows % 89 + n_tok)
+
+
+@pytest.mark.parametrize("name,in_dim", [("f16", 320), ("bf16", 256)])
+def test_gemm_dense_full_grid(name, in_dim):
+    run_some(name, 16500, in_dim, 17, seed=160)  # 32 tokens x 64 rows
+
+
+@pytest.mark.parametrize("name", GEMM_TYPES)
+@pytest.mark.parametrize("rows,n_tok", [(16400, 40), (32641, 40)])
+def test_gemm_full_grids_x_range(name, rows, n_tok):
+    # test_gemm_x_range's tokens, and ones below 2^-86, in the tiles of a full grid
+    in_dim = 768
+    x = oracle.normal(92, (n_tok, in_dim)).astype(np.float64)
+    ramp = np.logspace(-6, 5, in_dim // 128).repeat(128)
+    kinds = [1.0, 1e5, 1e-6, ramp, ramp[::-1], 1e-30, np.where(np.arange(in_dim) < 256, 1e-27, 1.0),
+             np.where(np.arange(in_dim) < 256, 0.0, 1e-30)]
+    for t in range(n_tok):
+        x[t] *= kinds[t % len(kinds)]
+    run_some(name, rows, in_dim, n_tok, seed=170, x=x.astype(np.float32))
