@@ -696,20 +696,41 @@ static void launch(const GemmArgs& a, hipStream_t st) {
     hipLaunchKernelGGL((qgemm_kernel<TY, TT, RT, WR>), dim3((unsigned)grid), dim3(512), 0, st, a);
 }
 
-// Tiles: 64 tokens (32 for a batch of at most 32), and 64 rows where they
-// still make a workgroup for every CU, else 32 (fewer rows raise the share of
-// x's staging, which every workgroup of a token block repeats; dense rows take
-// 32 beside 64 tokens, whose x leaves LDS for no more).
+// Tiles.  Up to 32 tokens: 32 x 32, or 32 x 64 where those still make a
+// workgroup for every CU (fewer rows raise the share of x's staging, which
+// every workgroup of a token block repeats).  Dense rows beside more tokens: 64
+// x 32, whose x leaves LDS for no more.  Block formats beside more: 64 tokens x
+// 32, 64 or 128 (qgemm_big.hip) rows.  A CU holds one workgroup, so a call
+// takes as many rounds as its grid has times 256, each about as long whatever
+// is in it.  us a round at in_dim 4096 (1024): 64 x 32 Q4_K 41 (16), Q6_K 40
+// (16), Q8_0 34 (14); 64 x 64 50 (20), 51 (20), 46 (18); 64 x 128 65 (23), 84
+// (29), 71 (23), and where the last token block is not whole 84 (27), 118 (37),
+// 98 (33).  The least rounds times that is taken; from 256 workgroups of 64 x
+// 128 on those always are.  us a call, 64 x 128 everywhere / 64 x 64 wherever it
+// made 256 workgroups / now: Q4_K 64 tokens x 12288 x 4096 65 / 79 / 49, 512 x
+// 3000 x 4096 68 / 95 / 66; Q6_K 128 x 6000 x 4096 84 / 76 / 50, 512 x 3000 x
+// 4096 86 / 96 / 87, 400 x 3000 x 4096 121 / 96 / 96.
 constexpr long kCus = 256;
-static bool fills(const GemmArgs& a, int tm, int tn) {
-    return ((long)a.n_tok + tm - 1) / tm * ((a.rows + tn - 1) / tn) >= kCus;
+static long blocks(const GemmArgs& a, int tm, int tn) {
+    return ((long)a.n_tok + tm - 1) / tm * ((a.rows + tn - 1) / tn);
+}
+// Rows of a block format's tile of 64 tokens.
+static int tile_rows(const GemmArgs& a, uint32_t type) {
+    if (blocks(a, 64, 128) >= kCus) return 128;
+    // in hundredths of a 64 x 32 round
+    const int big = a.n_tok % 64 ? (type == kGQ4K ? 200 : 290) : type == kGQ4K ? 160 : 205;
+    const int mid = type == kGQ4K ? 122 : type == kGQ6K ? 128 : 135;
+    auto rounds = [&](int tn) { return (blocks(a, 64, tn) + kCus - 1) / kCus; };
+    const long c32 = rounds(32) * 100, c64 = rounds(64) * mid;
+    if (std::min(c32, c64) > big) return 128;
+    return c64 < c32 ? 64 : 32;
 }
 template <int TY>
-static void launch_type(const GemmArgs& a, hipStream_t st) {
+static void launch_type(const GemmArgs& a, int tn, hipStream_t st) {
     if (a.n_tok <= 32) {
-        if (fills(a, 32, 64)) launch<TY, 1, 1, 2>(a, st);
+        if (blocks(a, 32, 64) >= kCus) launch<TY, 1, 1, 2>(a, st);
         else launch<TY, 1, 1, 1>(a, st);
-    } else if (!g_dense<TY>() && fills(a, 64, 64)) {
+    } else if (!g_dense<TY>() && tn == 64) {
         if constexpr (!g_dense<TY>()) launch<TY, 2, 1, 2>(a, st);
     } else {
         launch<TY, 2, 1, 1>(a, st);
@@ -742,15 +763,15 @@ lmx_status qgemm(const lmx_qmv_desc* d, const void* w, const float* x, float* y,
     a.row_bytes = (size_t)d->in_dim / be * bb;
     a.w_bytes = a.row_bytes * d->rows;
     if (((long)d->n_tok + 31) / 32 * (((long)d->rows + 31) / 32) > INT32_MAX) return LMX_E_SHAPE;
-    // 64 x 128 tiles where they fill the GPU (see qgemm_big.hip)
-    if (be > 1 && d->n_tok > 32 && fills(a, 64, 128)) return qgemm_big(d, w, x, y, st);
+    const int tn = be > 1 && d->n_tok > 32 ? tile_rows(a, d->type) : 32;
+    if (tn == 128) return qgemm_big(d, w, x, y, st);
     (void)hipGetLastError();
     switch (d->type) {
-        case kGF16: launch_type<kGF16>(a, st); break;
-        case kGBF16: launch_type<kGBF16>(a, st); break;
-        case kGQ4K: launch_type<kGQ4K>(a, st); break;
-        case kGQ6K: launch_type<kGQ6K>(a, st); break;
-        default: launch_type<kGQ8_0>(a, st); break;
+        case kGF16: launch_type<kGF16>(a, tn, st); break;
+        case kGBF16: launch_type<kGBF16>(a, tn, st); break;
+        case kGQ4K: launch_type<kGQ4K>(a, tn, st); break;
+        case kGQ6K: launch_type<kGQ6K>(a, tn, st); break;
+        default: launch_type<kGQ8_0>(a, tn, st); break;
     }
     LMX_CHECK_LAUNCH();
     return LMX_OK;

@@ -308,9 +308,9 @@ def test_dense_infinite_and_nan(name, n_tok):
             assert np.abs(got[t, f] - ref[t, f]).max() <= 3e-5 * np.abs(ref[t, f]).max(), t
 
 
-# ---- grids of a workgroup for every CU: 64 tokens x 64 rows, 64 x 128 (the
-# kernel of its own, qgemm_big.hip), and dense 32 tokens x 64 rows.  All rows
-# are computed; the first, some in the middle and the last are checked.
+# ---- large grids: 64 tokens x 64 rows, 64 x 128 (the kernel of its own,
+# qgemm_big.hip), and dense 32 tokens x 64 rows.  All rows are computed; the
+# first, some in the middle and the last are checked.
 def some_rows(rows):
     return sorted(set(list(range(140)) + list(range(rows // 2, rows // 2 + 70)) + list(range(rows - 140, rows))))
 
@@ -331,8 +331,9 @@ def run_some(name, rows, in_dim, n_tok, seed, x=None):
 @pytest.mark.parametrize("name,in_dim", [("q4_k", 256), ("q4_k", 768), ("q6_k", 256), ("q6_k", 768), ("q8_0", 128),
                                          ("q8_0", 384)])
 @pytest.mark.parametrize("rows,n_tok", [
-    (16400, 40), (16321, 64),                            # 64 x 64
-    (4090, 500), (32641, 33), (32768, 64), (8065, 257)])  # 64 x 128, whole and ragged
+    (16321, 64), (8200, 40), (4100, 190),                # 64 x 64
+    (4090, 500), (32641, 33), (32768, 64), (8065, 257),  # 64 x 128, whole and ragged,
+    (16400, 40), (3000, 512)])                           # and in grids that leave CUs over
 def test_gemm_full_grids(name, in_dim, rows, n_tok):
     run_some(name, rows, in_dim, n_tok, seed=140 + rows % 89 + n_tok)
 
@@ -343,7 +344,7 @@ def test_gemm_dense_full_grid(name, in_dim):
 
 
 @pytest.mark.parametrize("name", GEMM_TYPES)
-@pytest.mark.parametrize("rows,n_tok", [(16400, 40), (32641, 40)])
+@pytest.mark.parametrize("rows,n_tok", [(8200, 40), (32641, 40)])
 def test_gemm_full_grids_x_range(name, rows, n_tok):
     # test_gemm_x_range's tokens, and ones below 2^-86, in the tiles of a full grid
     in_dim = 768
