@@ -35,10 +35,11 @@
 // queries, us a call): head_dim 512, 16 heads on one kv head, 2048 tokens
 // 979 / 391 -> 149 / 124; 4096 tokens 3792 / 1482 -> 520 / 430 (531 / 640
 // TFLOP/s); head_dim 256, 16 heads on 8, window 1024, 1999 tokens at 3001
-// 92 / 79 -> 74 / 57; 4096 tokens, no window 305 / 228 -> 235 / 186.  What
+// 92 / 79 -> 78 / 60; 4096 tokens, no window 305 / 228 -> 235 / 186.  What
 // bounds it: with the transfers skipped a head_dim 512 call takes two thirds
-// of the time, without the MFMAs as long; the transfers run at about 28
-// bytes a cycle and CU, and overlap little of the scores and softmax.  Tried
+// of the time, without the MFMAs as long; the transfers move 10.5 TB/s of tiles
+// over all CUs (head_dim 512, 4096 f16-query tokens: 33 thousand of 128 KB in
+// 404 us), and overlap little of the scores and softmax.  Tried
 // and no faster: the two waves of a SIMD half a tile apart (ping-pong; at 512
 // it halves the tile and lost 25%), transfers dealt out between the MFMAs.
 #include <climits>

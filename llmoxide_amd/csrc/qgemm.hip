@@ -50,11 +50,12 @@
 //
 // Measured (in_dim 4096, us a call; before: 64 x 128 tiles with one wave kind
 // per stage for the block formats, four tokens a launch for dense rows):
-// 16 tokens x 4096 rows Q4_K 81 -> 26, Q6_K 116 -> 29, Q8_0 94 -> 23, bf16
-// 103 -> 26; 500 x 1024 rows 83 -> 40, 120 -> 38, 99 -> 34, 2577 -> 37; 64 x
-// 4096 rows bf16 433 -> 37.  What bounds it: a chunk's round trip (its x and W
-// loads are a chunk ahead, about 1.5 us) and x's staging (1.2 us of vector
-// work a chunk at 64 tokens), against 0.3 us of MFMAs at 64 x 32.
+// 16 tokens x 4096 rows Q4_K 81 -> 25, Q6_K 116 -> 29, Q8_0 94 -> 22, bf16
+// 103 -> 25; 500 x 1024 rows 83 -> 40, 120 -> 39, 99 -> 34, 2577 -> 36; 64 x
+// 4096 rows bf16 433 -> 36.  What bounds it: a workgroup's chunks come one after
+// the other, each a round trip (its x and W loads are a chunk ahead; 1.5 us at
+// 32 tokens) or x's staging (2.1 us a chunk at 64), with the vector unit busy 57
+// to 65% of the time and the matrix pipe 3 to 14%.
 #include <algorithm>
 #include <climits>
 
