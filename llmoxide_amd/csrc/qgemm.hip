@@ -7,15 +7,10 @@
 // 1083) and computes what its CPU reference dot_row computes
 // (crates/gguf/src/quant.rs:187-271), to fp32 accuracy:
 //
-//   Every block format is  w = s_g * q + o_g  over groups g of 16 or 32
-//   consecutive weights, q a small integer:
-//     Q4_K  q in [0, 15],     s = d * sc_g, o = -dmin * m_g  (groups of 32)
-//     Q6_K  q in [-32, 31],   s = d * sc_g, o = 0            (groups of 16)
-//     Q8_0  q in [-128, 127], s = d,        o = 0            (groups of 32)
+//   The block formats: qgemm.hpp.
 //   x, scaled (below), is split into f16 x_hi + x_lo, and all products run on
-//   v_mfma_f32_32x32x16_f16 with fp32 accumulation.  The
-//   integer scales go into the weight operand, where the vector unit pays for
-//   them once a weight instead of once a token: sc_g q of Q4_K is at most 945
+//   v_mfma_f32_32x32x16_f16 with fp32 accumulation.  The integer scales go
+//   into the weight operand, where the vector unit pays for them once a weight instead of once a token: sc_g q of Q4_K is at most 945
 //   and exact in f16; of Q6_K it is at most 4096 and exact as f16(sc_g q) plus
 //   a remainder (third product: remainder times x_hi).  Only d, one a
 //   super-block of 256, is applied to the fp32 sums (of a bf16 row, the power
@@ -59,12 +54,11 @@
 #include <algorithm>
 #include <climits>
 
-#include "common.hpp"
 #include "lds_dma.hpp"
+#include "qgemm.hpp"
 
 namespace lmx {
 
-enum GType { kGF16 = 1, kGQ8_0 = 8, kGQ4K = 12, kGQ6K = 14, kGBF16 = 30 };
 template <int TY>
 constexpr bool g_dense() { return TY == kGF16 || TY == kGBF16; }
 
@@ -109,12 +103,6 @@ __device__ __forceinline__ float wave_max64(float x) {
     const float r2 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 32));
     const float r3 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 48));
     return fmaxf(fmaxf(r0, r1), fmaxf(r2, r3));
-}
-// Sum over each aligned group of 8 lanes; every lane of the group gets it.
-__device__ __forceinline__ float sum8(float x) {
-    x += dpp<0xB1>(x);   // quad_perm [1,0,3,2]
-    x += dpp<0x4E>(x);   // quad_perm [2,3,0,1]
-    return x + dpp<0x141>(x);  // row_half_mirror: lane i with 7 - i of its 8
 }
 
 __device__ __forceinline__ f16x2 as_h2(uint32_t x) { return __builtin_bit_cast(f16x2, x); }
