@@ -284,16 +284,29 @@ def _ptr(t) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
+def _stream_calls(torch):
+    """(handle of a device's current stream, current device), by torch's raw
+    calls where it has them: a call of a few microseconds notices the
+    torch.cuda.Stream object that current_stream() makes."""
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None:
+        return lambda dev: torch.cuda.current_stream(dev).cuda_stream, torch.cuda.current_device
+    return raw, getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
+
+
+_calls = None
+
+
 def _stream(stream) -> Optional[int]:
     if stream is not None:
         return stream.cuda_stream
     torch = _torch()
-    # the raw handle alone, where this torch has it: a call of a few microseconds
-    # notices the torch.cuda.Stream object that current_stream() makes for it
-    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-    if raw is None:
+    if not torch.cuda.is_initialized():
         return torch.cuda.current_stream().cuda_stream
-    return raw(torch.cuda.current_device())
+    global _calls
+    if _calls is None:
+        _calls = _stream_calls(torch)
+    return _calls[0](_calls[1]())
 
 
 def _dt(t) -> int:

@@ -403,14 +403,16 @@ def test_padded_head_dims_validate_and_size_their_copies():
                                      lmx.F16, FAKE + (1 << 24), None, 0, None) == lmx.Status.E_UNSUPPORTED
 
 
-def test_current_stream_without_the_raw_handle(monkeypatch):
-    """torch builds without the private raw-handle call are asked for the
-    stream object; the handle is the current device's otherwise."""
+def test_current_stream_without_the_raw_calls():
+    """A torch without the private raw-handle call, or without the private
+    device call beside it, is asked through its public ones."""
     from types import SimpleNamespace
-    cuda = SimpleNamespace(current_stream=lambda: SimpleNamespace(cuda_stream=77), current_device=lambda: 3)
-    monkeypatch.setattr(lmx, "_torch", lambda: SimpleNamespace(_C=SimpleNamespace(), cuda=cuda))
-    assert lmx._stream(None) == 77
-    raw = SimpleNamespace(_cuda_getCurrentRawStream=lambda dev: 100 + dev)
-    monkeypatch.setattr(lmx, "_torch", lambda: SimpleNamespace(_C=raw, cuda=cuda))
-    assert lmx._stream(None) == 103
+    cuda = SimpleNamespace(current_stream=lambda dev: SimpleNamespace(cuda_stream=70 + dev), current_device=lambda: 3)
+
+    def handle(**c):
+        stream_of, device = lmx._stream_calls(SimpleNamespace(_C=SimpleNamespace(**c), cuda=cuda))
+        return stream_of(device())
+    assert handle() == 73
+    assert handle(_cuda_getCurrentRawStream=lambda dev: 100 + dev) == 103
+    assert handle(_cuda_getCurrentRawStream=lambda dev: 100 + dev, _cuda_getDevice=lambda: 5) == 105
     assert lmx._stream(SimpleNamespace(cuda_stream=5)) == 5
